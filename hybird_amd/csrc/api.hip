@@ -174,6 +174,8 @@ struct hyb_dem {
     bool inited = false;
     hipStream_t stream = nullptr;
     int64_t substeps = 0;
+    bool wholeStep = false;  // a DEM step is one launch (launch_dem_run); otherwise three per sub-step
+    bool entStale = false;   // the per-element pair entries of that launch do not belong to the current lists
     ErrWord err;             // device-side failures of the DEM kernels
     std::vector<Blk> saved;  // persistent device state
     // MercuryDPM-format saving (DEM.cpp:355-360, 1131-1146): captures of the
@@ -331,8 +333,8 @@ static int dem_pending(const hyb_dem* d) {
         return fail(HYB_E_NUMERIC, "DEM: non-finite element velocity; the DEM stopped at that sub-step");
     return fail(HYB_E_CAPACITY, "DEM device error " + std::to_string(e) +
                                     " (1/4: ghost or pair capacity, 2: particle outside the cell grid, 3: stencil outside"
-                                    " the cell table, 5: more than 16 objects near one particle); the DEM stopped at"
-                                    " that sub-step");
+                                    " the cell table, 5: more than 16 objects near one particle, 7: the workgroups of a"
+                                    " DEM step did not meet); the DEM stopped at that sub-step");
 }
 
 static int lb_pending(const hyb_lb* l) {
@@ -463,6 +465,13 @@ int hyb_dem_init_lattice(hyb_dem* d, const int32_t boundary[6], const int32_t lb
     li.unit = make_units(unitLength, unitTime, unitDensity);
     for (int k = 0; k < 3; ++k) li.lbF[k] = lbF[k];
     return dem_init(d, li);
+}
+
+// Barrier words and counter of the whole-step kernel as before its first launch.
+static int dem_run_reset(hyb_dem* d) {
+    HIPCHK(hipMemsetAsync(d->b.runSlots, 0xFF, 24 * (size_t)dem_run_workgroups(d->p), d->stream));
+    HIPCHK(hipMemsetAsync(d->b.st2, 0, sizeof(DEMRunState), d->stream));
+    return HYB_OK;
 }
 
 static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
@@ -726,6 +735,16 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
         (rc = dalloc(&b.wcf, (size_t)std::max(P, 1) * wall_slots(p))))
         return rc;
     HIPCHK(hipMemset(b.wcf, 0, sizeof(ContactForce) * (size_t)std::max(P, 1) * wall_slots(p)));
+    d->wholeStep = dem_run_fits(p);
+    if (d->wholeStep) {
+        const size_t wg = (size_t)dem_run_workgroups(p);
+        if ((rc = dalloc(&b.runSlots, 3 * wg)) || (rc = dalloc(&b.st2, 1)) || (rc = dalloc(&b.runCount, RUN_COUNTS * wg)) ||
+            (rc = dalloc(&b.xch, 2 * RUN_REC * (size_t)P)) || (rc = dalloc(&b.pairCount, (size_t)P)) ||
+            (rc = dalloc(&b.csrTmp, 2 * (size_t)p.pairCap)) || (rc = dalloc(&b.ent, 2 * (size_t)p.pairCap)) ||
+            (p.spring && (rc = dalloc(&b.entHist, 6 * (size_t)p.pairCap))))
+            return rc;
+        if ((rc = dem_run_reset(d))) return rc;
+    }
     if (p.allWalls) {
         if ((rc = ralloc(R, "nearWallMask", &b.nearWallMask, (size_t)std::max(P, 1)))) return rc;
         HIPCHK(hipMemset(b.nearWallMask, 0, sizeof(uint32_t) * (size_t)std::max(P, 1)));
@@ -763,6 +782,19 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
         HIPCHK(hipMemcpy(objs, d->objects.data(), sizeof(ObjDev) * (size_t)p.nobj, hipMemcpyHostToDevice));
         b.objs = objs;
     }
+    if (d->wholeStep) {  // every buffer is set by now
+        DEMRunArgs* ra = nullptr;
+        if ((rc = dalloc(&ra, 1))) return rc;
+        b.runArgs = ra;
+        DEMRunArgs host;
+        host.p = p;
+        host.b = b;
+        HIPCHK(hipMemcpyAsync(ra, &host, sizeof(host), hipMemcpyHostToDevice, d->stream));
+        HIPCHK(hipStreamSynchronize(d->stream));
+    }
+    // the uploads above (hipMemcpy, hipMemset) went to the null stream, which the handle's non-blocking stream
+    // does not wait for, and a copy from pageable memory may return before it has reached the device
+    HIPCHK(hipStreamSynchronize(nullptr));
     HIPCHK(hipMemcpyAsync(b.el, el.data(), el.size() * sizeof(double), hipMemcpyHostToDevice, d->stream));
     DEMState st;
     std::memset(&st, 0, sizeof(st));
@@ -776,7 +808,9 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
     HIPCHK(hipMemsetAsync(b.ghostOfCount, 0, sizeof(int) * std::max(P, 1), d->stream));
     if (P) {
         launch_dem_particles(p, b, d->stream);   // generateParticles (elmt.cpp:122-137)
-        launch_dem_rebuild(p, b, 1, d->stream);  // evalNeighborTable at init (DEM.cpp:258-262)
+        // evalNeighborTable at init (DEM.cpp:258-262)
+        if (d->wholeStep) launch_dem_run(p, b, 0, 1, d->stream);
+        else launch_dem_rebuild(p, b, 1, d->stream);
         launch_dem_predict(p, b, d->stream);     // the first sub-step's predictor
     }
     HIPCHK(hipGetLastError());
@@ -816,6 +850,7 @@ int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
     if (!d || !d->inited) return fail(HYB_E_STATE, "hyb_dem_step before hyb_dem_init");
     if (int rc = dem_pending(d)) return rc;
     d->saveEvents.clear();
+    const bool whole = d->wholeStep && !d->saveCount;
     for (int it = 0; it < d->multiStep; ++it) {
         d->demTimeStep++;
         d->demTime += d->deltat;
@@ -825,7 +860,7 @@ int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
             if (slot >= d->saveSlots) return fail(HYB_E_STATE, "hyb_dem_step: more saving sub-steps than slots");
             d->saveEvents.emplace_back(d->demTime, d->demTimeStep);
         }
-        if (d->P) {
+        if (d->P && !whole) {
             launch_dem_rebuild(d->p, d->b, 0, d->stream);
             if (save) {
                 const size_t P = (size_t)d->P;
@@ -840,8 +875,14 @@ int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
                 launch_dem_pairs(d->p, d->b, d->stream);
                 launch_dem_gather(d->p, d->b, d->stream);
             }
+            d->entStale = true;
         }
         d->substeps++;
+    }
+    if (d->P && whole && d->multiStep > 0) {
+        if (d->entStale) launch_dem_entries(d->p, d->b, d->stream);
+        d->entStale = false;
+        launch_dem_run(d->p, d->b, d->multiStep, 0, d->stream);
     }
     HIPCHK(hipGetLastError());
     return HYB_OK;
@@ -858,8 +899,11 @@ int hyb_dem_destroy(hyb_dem* d) {
     dfree(b.wcf); dfree(b.ocf); dfree(b.nearCyl);
     dfree(b.hist); dfree(b.whist); dfree(b.histOld); dfree(b.pairsOld); dfree(b.csrOffOld); dfree(b.csrOld);
     dfree(b.ghostIndexOld);
+    dfree(b.runSlots); dfree(b.st2); dfree(b.runCount); dfree(b.xch); dfree(b.pairCount); dfree(b.csrTmp); dfree(b.ent);
+    dfree(b.entHist);
     dfree(b.pelem); dfree(b.efirst); dfree(b.pproto); dfree(b.pcor); dfree(b.ppred); dfree(b.pmn);
     if (b.objs) (void)hipFree((void*)b.objs);
+    if (b.runArgs) (void)hipFree((void*)b.runArgs);
     save_free(d);
     errword_free(d->err);
     delete d;
@@ -1086,6 +1130,7 @@ int hyb_lb_init(hyb_lb* l, hyb_dem* d) {  // LB.cpp:190-219
         for (int z = 0; z < l->Z; ++z)
             for (int k = 0; k < 3; ++k) m3[k] = std::max(m3[k], mz[3 * z + k]);
         HIPCHK(hipMemcpy(l->maxXYZ, m3, sizeof(m3), hipMemcpyHostToDevice));
+        HIPCHK(hipStreamSynchronize(nullptr));  // the handle's stream does not wait for the null stream
     }
     HIPCHK(hipMemsetAsync(l->f[0], 0, l->popBytes(), s));
     HIPCHK(hipMemsetAsync(l->f[1], 0, l->popBytes(), s));
@@ -2298,8 +2343,11 @@ int hyb_state_load(hyb_lb* l, hyb_dem* d, const char* path) {
             return rc;
         }
         errword_clear(d->err);
+        d->entStale = true;
+        if (d->wholeStep && (rc = dem_run_reset(d))) return rc;
         d->demTime = s.demTime; d->demTimeStep = s.demTimeStep; d->substeps = s.substeps;
     }
+    HIPCHK(hipStreamSynchronize(nullptr));  // the handles' stream does not wait for the null stream's copies
     return HYB_OK;
 }
 

@@ -58,8 +58,9 @@ __host__ __device__ inline int wall_slots(const DEMParams& p) { return p.allWall
 
 // DEMState::error codes: 1 ghost capacity, 2 particle outside the cell grid,
 // 3 stencil outside the cell table, 4 pair capacity, 5 more than NEAR_OBJ objects
-// near one particle, 6 non-finite element velocity.
+// near one particle, 6 non-finite element velocity, 7 the workgroups of a DEM step did not meet.
 constexpr int DEM_ERR_NUMERIC = 6;
+constexpr int DEM_ERR_BARRIER = 7;
 
 // Objects a particle can have in range at once (a rebuild that finds more
 // reports DEMState::error 5).
@@ -141,10 +142,32 @@ struct DEMBuffers {
     double* pcor;          // [P][9]
     double* ppred;         // [P][9]
     double* pmn;           // [2 * pairCap][3]
+    // the whole-step kernel (dem_run.hip): barrier words [3][workgroups] (all ones: empty), which set comes next,
+    // counts per workgroup [workgroups][RUN_COUNTS], exchange records [2][P][RUN_REC], pairs per particle [P],
+    // unsorted per-particle pair lists and per element its pairs in order (and their springs) [2 * pairCap]
+    unsigned long long* runSlots;
+    struct DEMRunState* st2;
+    int* runCount;
+    double* xch;
+    int* pairCount;
+    uint32_t* csrTmp;
+    uint4* ent;
+    double* entHist;
+    const struct DEMRunArgs* runArgs;  // the parameters and buffers in device memory (for its rebuild)
     int scap;
     int ncells;
     int W;                 // ncells * 14
 };
+
+struct DEMRunState {
+    unsigned barriers;
+};
+struct DEMRunArgs {
+    DEMParams p;
+    DEMBuffers b;
+};
+constexpr int RUN_COUNTS = 8;
+constexpr int RUN_REC = 12;  // position, radius, velocity, mass, angular velocity, unused
 
 // Increments one contact adds to one element: the normal force (applied when
 // flag & 1), the normal-force moment of an element of size > 1 (flag & 4, held
@@ -188,6 +211,13 @@ void launch_dem_rebuild(const DEMParams& p, const DEMBuffers& b, int force, hipS
 // per-element gather (corrector, next predictor).
 void launch_dem_pairs(const DEMParams& p, const DEMBuffers& b, hipStream_t s);
 void launch_dem_gather(const DEMParams& p, const DEMBuffers& b, hipStream_t s);
+// The same sub-steps, rebuilds included, in one launch (force: only an unconditional rebuild, as at initialisation).
+// dem_run_fits: whether its workgroups (dem_run_workgroups) can all be resident at once on this device.
+int dem_run_workgroups(const DEMParams& p);
+bool dem_run_fits(const DEMParams& p);
+void launch_dem_run(const DEMParams& p, const DEMBuffers& b, int nsub, int force, hipStream_t s);
+// DEMBuffers::ent from the pair lists (after a rebuild by launch_dem_rebuild or a state load).
+void launch_dem_entries(const DEMParams& p, const DEMBuffers& b, hipStream_t s);
 void launch_dem_predict(const DEMParams& p, const DEMBuffers& b, hipStream_t s);
 // Particle positions, velocities and radius vectors of every particle from its
 // element's corrected and predicted state (multi-sphere elements only).
