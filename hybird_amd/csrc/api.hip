@@ -21,6 +21,7 @@
 #include "fs_kernels.h"
 #include "hybird_amd.h"
 #include "lb_kernels.h"
+#include "view_kernels.h"
 
 using namespace hyb;
 
@@ -90,6 +91,48 @@ void dfree(T*& p) {
     p = nullptr;
 }
 
+// Device memory of one handle, freed as a whole: requests are cut from slabs of `slab` bytes, larger ones get a
+// slab of their own. A handle has some sixty buffers, and every hipFree costs about 70 us (7 ms to destroy a small
+// simulation).
+constexpr size_t ARENA_ALIGN = 256;
+struct Arena {
+    std::vector<void*> slabs;
+    char* next = nullptr;
+    size_t left = 0, slab = (size_t)4 << 20;
+    int take(void** p, size_t bytes) {
+        *p = nullptr;
+        if (bytes == 0) return HYB_OK;
+        bytes = (bytes + ARENA_ALIGN - 1) / ARENA_ALIGN * ARENA_ALIGN;
+        if (bytes > left) {
+            const size_t size = std::max(bytes, slab);
+            void* q = nullptr;
+            HIPCHK(hipMalloc(&q, size));
+            slabs.push_back(q);
+            if (size > slab) {  // the rest of the current slab stays in use
+                *p = q;
+                return HYB_OK;
+            }
+            next = (char*)q;
+            left = size;
+        }
+        *p = next;
+        next += bytes;
+        left -= bytes;
+        return HYB_OK;
+    }
+    void release() {
+        for (void* q : slabs) (void)hipFree(q);
+        slabs.clear();
+        next = nullptr;
+        left = 0;
+    }
+};
+
+template <class T>
+int dalloc(Arena& a, T** p, size_t count) {
+    return a.take((void**)p, count * sizeof(T));
+}
+
 // A device buffer that belongs to a handle's persistent state (written by
 // hyb_state_save, restored by hyb_state_load).
 struct Blk {
@@ -102,6 +145,13 @@ struct Blk {
 template <class T>
 int ralloc(std::vector<Blk>& reg, const char* name, T** p, size_t count) {
     const int rc = dalloc(p, count);
+    if (rc == HYB_OK && *p) reg.push_back(Blk{name, (void*)*p, count * sizeof(T)});
+    return rc;
+}
+
+template <class T>
+int ralloc(Arena& a, std::vector<Blk>& reg, const char* name, T** p, size_t count) {
+    const int rc = dalloc(a, p, count);
     if (rc == HYB_OK && *p) reg.push_back(Blk{name, (void*)*p, count * sizeof(T)});
     return rc;
 }
@@ -177,7 +227,9 @@ struct hyb_dem {
     bool wholeStep = false;  // a DEM step is one launch (launch_dem_run); otherwise three per sub-step
     bool entStale = false;   // the per-element pair entries of that launch do not belong to the current lists
     ErrWord err;             // device-side failures of the DEM kernels
+    Arena arena;             // every device buffer below except the saving ones
     std::vector<Blk> saved;  // persistent device state
+    double* view = nullptr;  // packed host view [E][24]
     // MercuryDPM-format saving (DEM.cpp:355-360, 1131-1146): captures of the
     // saving sub-steps of the last hyb_dem_step, one slot each
     int saveCount = 0;
@@ -254,6 +306,7 @@ struct hyb_lb {
     // reverse pass's buffers (states of one interval, two adjoint population
     // buffers, dL/dF, tau partials) and the device time of both loops
     int adjSteps = -1, adjEvery = 0;
+    Arena adjArena;
     std::vector<void*> adjCk;
     std::vector<void*> adjSeg;
     double* adjLam[2] = {nullptr, nullptr};
@@ -267,7 +320,10 @@ struct hyb_lb {
     double profMs = 0.0;
     int64_t profLaunches = 0;
     ErrWord err;             // device-side failures of the LB kernels
+    Arena arena;             // device buffers except those made on demand
     std::vector<Blk> saved;  // persistent device state
+    void* view = nullptr;    // packed part of a host view or input (viewBytes, at most VIEW_BYTES)
+    size_t viewBytes = 0;
 
     bool varVisc() const { return nonNewtonian || turbulenceOn || frictional; }
     bool hasSlip() const {
@@ -719,41 +775,43 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
     errword_clear(d->err);
     p.herr = d->err.dev;
     std::vector<Blk>& R = d->saved;
+    Arena& A = d->arena;
     R.clear();
-    if ((rc = ralloc(R, "el", &b.el, el.size())) || (rc = ralloc(R, "st", &b.st, 1)) ||
-        (rc = ralloc(R, "ghostIndex", &b.ghostIndex, p.Gcap)) || (rc = ralloc(R, "ghostVec", &b.ghostVec, 3 * (size_t)p.Gcap)) ||
-        (rc = ralloc(R, "pairs", &b.pairs, 2 * (size_t)p.pairCap)) || (rc = ralloc(R, "nearWall", &b.nearWall, std::max(P, 1))) ||
-        (rc = ralloc(R, "cellTable", &b.cellTable, (size_t)scap + b.ncells)) || (rc = ralloc(R, "cellOf", &b.cellOf, scap)) ||
-        (rc = ralloc(R, "cellCount", &b.cellCount, b.ncells + 1)) ||
-        (rc = dalloc(&b.work, (size_t)std::max(std::max(b.W, scap), std::max(p.pairCap, b.ncells + 1)) + 1)) ||
-        (rc = ralloc(R, "csrOff", &b.csrOff, (size_t)P + 1)) || (rc = ralloc(R, "csr", &b.csr, 2 * (size_t)p.pairCap)) ||
-        (rc = dalloc(&b.cursor, scap)) || (rc = dalloc(&b.spos, 4 * (size_t)scap)) || (rc = ralloc(R, "ghostOfCount", &b.ghostOfCount, std::max(P, 1))) ||
-        (rc = ralloc(R, "ghostOf", &b.ghostOf, 8 * (size_t)std::max(P, 1))) ||
-        (rc = ralloc(R, "side", &b.side, 3 * (size_t)std::max(P, 1))) || (rc = ralloc(R, "ghostB", &b.ghostB, p.Gcap)) ||
-        (rc = ralloc(R, "posI", &b.posI, p.pairCap)) || (rc = ralloc(R, "posJ", &b.posJ, p.pairCap)) ||
-        (rc = dalloc(&b.prec, 2 * (size_t)p.pairCap)) || (rc = ralloc(R, "vmax", &b.vmax, 1)) || (rc = dalloc(&b.energy, 6)) ||
-        (rc = dalloc(&b.wcf, (size_t)std::max(P, 1) * wall_slots(p))))
+    A.release();
+    if ((rc = ralloc(A, R, "el", &b.el, el.size())) || (rc = ralloc(A, R, "st", &b.st, 1)) ||
+        (rc = ralloc(A, R, "ghostIndex", &b.ghostIndex, p.Gcap)) || (rc = ralloc(A, R, "ghostVec", &b.ghostVec, 3 * (size_t)p.Gcap)) ||
+        (rc = ralloc(A, R, "pairs", &b.pairs, 2 * (size_t)p.pairCap)) || (rc = ralloc(A, R, "nearWall", &b.nearWall, std::max(P, 1))) ||
+        (rc = ralloc(A, R, "cellTable", &b.cellTable, (size_t)scap + b.ncells)) || (rc = ralloc(A, R, "cellOf", &b.cellOf, scap)) ||
+        (rc = ralloc(A, R, "cellCount", &b.cellCount, b.ncells + 1)) ||
+        (rc = dalloc(A, &b.work, (size_t)std::max(std::max(b.W, scap), std::max(p.pairCap, b.ncells + 1)) + 1)) ||
+        (rc = ralloc(A, R, "csrOff", &b.csrOff, (size_t)P + 1)) || (rc = ralloc(A, R, "csr", &b.csr, 2 * (size_t)p.pairCap)) ||
+        (rc = dalloc(A, &b.cursor, scap)) || (rc = dalloc(A, &b.spos, 4 * (size_t)scap)) || (rc = ralloc(A, R, "ghostOfCount", &b.ghostOfCount, std::max(P, 1))) ||
+        (rc = ralloc(A, R, "ghostOf", &b.ghostOf, 8 * (size_t)std::max(P, 1))) ||
+        (rc = ralloc(A, R, "side", &b.side, 3 * (size_t)std::max(P, 1))) || (rc = ralloc(A, R, "ghostB", &b.ghostB, p.Gcap)) ||
+        (rc = ralloc(A, R, "posI", &b.posI, p.pairCap)) || (rc = ralloc(A, R, "posJ", &b.posJ, p.pairCap)) ||
+        (rc = dalloc(A, &b.prec, 2 * (size_t)p.pairCap)) || (rc = ralloc(A, R, "vmax", &b.vmax, 1)) || (rc = dalloc(A, &b.energy, 6)) ||
+        (rc = dalloc(A, &b.wcf, (size_t)std::max(P, 1) * wall_slots(p))))
         return rc;
     HIPCHK(hipMemset(b.wcf, 0, sizeof(ContactForce) * (size_t)std::max(P, 1) * wall_slots(p)));
     d->wholeStep = dem_run_fits(p);
     if (d->wholeStep) {
         const size_t wg = (size_t)dem_run_workgroups(p);
-        if ((rc = dalloc(&b.runSlots, 3 * wg)) || (rc = dalloc(&b.st2, 1)) || (rc = dalloc(&b.runCount, RUN_COUNTS * wg)) ||
-            (rc = dalloc(&b.xch, 2 * RUN_REC * (size_t)P)) || (rc = dalloc(&b.pairCount, (size_t)P)) ||
-            (rc = dalloc(&b.csrTmp, 2 * (size_t)p.pairCap)) || (rc = dalloc(&b.ent, 2 * (size_t)p.pairCap)) ||
-            (p.spring && (rc = dalloc(&b.entHist, 6 * (size_t)p.pairCap))))
+        if ((rc = dalloc(A, &b.runSlots, 3 * wg)) || (rc = dalloc(A, &b.st2, 1)) || (rc = dalloc(A, &b.runCount, RUN_COUNTS * wg)) ||
+            (rc = dalloc(A, &b.xch, 2 * RUN_REC * (size_t)P)) || (rc = dalloc(A, &b.pairCount, (size_t)P)) ||
+            (rc = dalloc(A, &b.csrTmp, 2 * (size_t)p.pairCap)) || (rc = dalloc(A, &b.ent, 2 * (size_t)p.pairCap)) ||
+            (p.spring && (rc = dalloc(A, &b.entHist, 6 * (size_t)p.pairCap))))
             return rc;
         if ((rc = dem_run_reset(d))) return rc;
     }
     if (p.allWalls) {
-        if ((rc = ralloc(R, "nearWallMask", &b.nearWallMask, (size_t)std::max(P, 1)))) return rc;
+        if ((rc = ralloc(A, R, "nearWallMask", &b.nearWallMask, (size_t)std::max(P, 1)))) return rc;
         HIPCHK(hipMemset(b.nearWallMask, 0, sizeof(uint32_t) * (size_t)std::max(P, 1)));
     }
-    if (p.ncyl && (rc = ralloc(R, "nearCyl", &b.nearCyl, (size_t)std::max(P, 1)))) return rc;
+    if (p.ncyl && (rc = ralloc(A, R, "nearCyl", &b.nearCyl, (size_t)std::max(P, 1)))) return rc;
     if (p.clumps) {
-        if ((rc = dalloc(&b.pelem, (size_t)P)) || (rc = dalloc(&b.efirst, (size_t)NE + 1)) ||
-            (rc = dalloc(&b.pproto, 3 * (size_t)P)) || (rc = ralloc(R, "pcor", &b.pcor, 9 * (size_t)P)) ||
-            (rc = ralloc(R, "ppred", &b.ppred, 9 * (size_t)P)) || (rc = dalloc(&b.pmn, 6 * (size_t)p.pairCap)))
+        if ((rc = dalloc(A, &b.pelem, (size_t)P)) || (rc = dalloc(A, &b.efirst, (size_t)NE + 1)) ||
+            (rc = dalloc(A, &b.pproto, 3 * (size_t)P)) || (rc = ralloc(A, R, "pcor", &b.pcor, 9 * (size_t)P)) ||
+            (rc = ralloc(A, R, "ppred", &b.ppred, 9 * (size_t)P)) || (rc = dalloc(A, &b.pmn, 6 * (size_t)p.pairCap)))
             return rc;
         HIPCHK(hipMemcpy(b.pelem, pelem.data(), sizeof(int) * pelem.size(), hipMemcpyHostToDevice));
         HIPCHK(hipMemcpy(b.efirst, efirst.data(), sizeof(int) * efirst.size(), hipMemcpyHostToDevice));
@@ -761,10 +819,10 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
     }
     if (p.spring) {
         const size_t Pm = (size_t)std::max(P, 1), Wm = Pm * (size_t)wall_slots(p);  // a spring per wall slot
-        if ((rc = ralloc(R, "hist", &b.hist, 3 * (size_t)p.pairCap)) || (rc = ralloc(R, "whist", &b.whist, 4 * Wm)) ||
-            (rc = dalloc(&b.histOld, 3 * (size_t)p.pairCap)) || (rc = dalloc(&b.pairsOld, 2 * (size_t)p.pairCap)) ||
-            (rc = dalloc(&b.csrOffOld, Pm + 1)) || (rc = dalloc(&b.csrOld, 2 * (size_t)p.pairCap)) ||
-            (rc = dalloc(&b.ghostIndexOld, (size_t)p.Gcap)))
+        if ((rc = ralloc(A, R, "hist", &b.hist, 3 * (size_t)p.pairCap)) || (rc = ralloc(A, R, "whist", &b.whist, 4 * Wm)) ||
+            (rc = dalloc(A, &b.histOld, 3 * (size_t)p.pairCap)) || (rc = dalloc(A, &b.pairsOld, 2 * (size_t)p.pairCap)) ||
+            (rc = dalloc(A, &b.csrOffOld, Pm + 1)) || (rc = dalloc(A, &b.csrOld, 2 * (size_t)p.pairCap)) ||
+            (rc = dalloc(A, &b.ghostIndexOld, (size_t)p.Gcap)))
             return rc;
         HIPCHK(hipMemset(b.hist, 0, 3 * sizeof(double) * (size_t)p.pairCap));
         std::vector<double> wh(4 * Wm, 0.0);
@@ -773,18 +831,19 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
     }
     if (p.nobj) {
         ObjDev* objs = nullptr;
-        if ((rc = ralloc(R, "objs", &objs, (size_t)p.nobj)) ||
-            (rc = ralloc(R, "nearObj", &b.nearObj, (size_t)P * NEAR_OBJ)) ||
-            (rc = ralloc(R, "nearObjCount", &b.nearObjCount, (size_t)P)) ||
-            (rc = dalloc(&b.ocf, (size_t)std::max(P, 1) * NEAR_OBJ)))
+        if ((rc = ralloc(A, R, "objs", &objs, (size_t)p.nobj)) ||
+            (rc = ralloc(A, R, "nearObj", &b.nearObj, (size_t)P * NEAR_OBJ)) ||
+            (rc = ralloc(A, R, "nearObjCount", &b.nearObjCount, (size_t)P)) ||
+            (rc = dalloc(A, &b.ocf, (size_t)std::max(P, 1) * NEAR_OBJ)))
             return rc;
         HIPCHK(hipMemset(b.ocf, 0, sizeof(ContactForce) * (size_t)std::max(P, 1) * NEAR_OBJ));
         HIPCHK(hipMemcpy(objs, d->objects.data(), sizeof(ObjDev) * (size_t)p.nobj, hipMemcpyHostToDevice));
         b.objs = objs;
     }
+    if ((rc = dalloc(A, &d->view, 24 * (size_t)std::max(NE, 1)))) return rc;
     if (d->wholeStep) {  // every buffer is set by now
         DEMRunArgs* ra = nullptr;
-        if ((rc = dalloc(&ra, 1))) return rc;
+        if ((rc = dalloc(A, &ra, 1))) return rc;
         b.runArgs = ra;
         DEMRunArgs host;
         host.p = p;
@@ -891,19 +950,7 @@ int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
 int hyb_dem_destroy(hyb_dem* d) {
     if (!d) return HYB_OK;
     if (d->stream) (void)hipStreamSynchronize(d->stream);
-    DEMBuffers& b = d->b;
-    dfree(b.el); dfree(b.st); dfree(b.ghostIndex); dfree(b.ghostVec); dfree(b.pairs); dfree(b.nearWall); dfree(b.nearWallMask);
-    dfree(b.cellTable); dfree(b.cellOf); dfree(b.cellCount); dfree(b.work); dfree(b.csrOff); dfree(b.csr);
-    dfree(b.cursor); dfree(b.spos); dfree(b.ghostOfCount); dfree(b.ghostOf); dfree(b.side); dfree(b.ghostB);
-    dfree(b.posI); dfree(b.posJ); dfree(b.prec); dfree(b.vmax); dfree(b.energy); dfree(b.nearObj); dfree(b.nearObjCount);
-    dfree(b.wcf); dfree(b.ocf); dfree(b.nearCyl);
-    dfree(b.hist); dfree(b.whist); dfree(b.histOld); dfree(b.pairsOld); dfree(b.csrOffOld); dfree(b.csrOld);
-    dfree(b.ghostIndexOld);
-    dfree(b.runSlots); dfree(b.st2); dfree(b.runCount); dfree(b.xch); dfree(b.pairCount); dfree(b.csrTmp); dfree(b.ent);
-    dfree(b.entHist);
-    dfree(b.pelem); dfree(b.efirst); dfree(b.pproto); dfree(b.pcor); dfree(b.ppred); dfree(b.pmn);
-    if (b.objs) (void)hipFree((void*)b.objs);
-    if (b.runArgs) (void)hipFree((void*)b.runArgs);
+    d->arena.release();
     save_free(d);
     errword_free(d->err);
     delete d;
@@ -990,37 +1037,37 @@ static int lb_alloc(hyb_lb* l, int slotCap) {
     const size_t pb = l->popBytes();
     std::vector<Blk>& R = l->saved;
     R.clear();
-    HIPCHK(hipMalloc(&l->f[0], pb));
-    HIPCHK(hipMalloc(&l->f[1], pb));
+    Arena& A = l->arena;
+    A.release();
+    if ((rc = A.take(&l->f[0], pb)) || (rc = A.take(&l->f[1], pb))) return rc;
     R.push_back(Blk{"f0", l->f[0], pb});
     R.push_back(Blk{"f1", l->f[1], pb});
-    if ((rc = ralloc(R, "type", &l->type, N)) || (rc = ralloc(R, "link", &l->link, N)) ||
-        (rc = ralloc(R, "solid", &l->solid, N)) ||
-        (rc = dalloc(&l->maxXYZ, 3 * (size_t)l->Z)) || (rc = dalloc(&l->dcount, (size_t)l->Z + 2)) ||
-        (rc = dalloc(&l->nslots, 2)))
+    if ((rc = ralloc(A, R, "type", &l->type, N)) || (rc = ralloc(A, R, "link", &l->link, N)) ||
+        (rc = ralloc(A, R, "solid", &l->solid, N)) ||
+        (rc = dalloc(A, &l->maxXYZ, 3 * (size_t)l->Z)) || (rc = dalloc(A, &l->dcount, (size_t)l->Z + 2)) ||
+        (rc = dalloc(A, &l->nslots, 2)))
         return rc;
-    if (l->varVisc() && (rc = ralloc(R, "visc", &l->visc, N))) return rc;
-    if (l->hasSlip() && (rc = ralloc(R, "slipw", &l->slipw, N))) return rc;
+    if (l->varVisc() && (rc = ralloc(A, R, "visc", &l->visc, N))) return rc;
+    if (l->hasSlip() && (rc = ralloc(A, R, "slipw", &l->slipw, N))) return rc;
     if (l->freeSurface) {
         FSBuffers& b = l->fsb;
         const size_t eb = l->prec == Prec::F64 ? 8 : 4;
-        HIPCHK(hipMalloc(&b.rho[0], eb * N));
-        HIPCHK(hipMalloc(&b.rho[1], eb * N));
+        if ((rc = A.take(&b.rho[0], eb * N)) || (rc = A.take(&b.rho[1], eb * N))) return rc;
         R.push_back(Blk{"rho0", b.rho[0], eb * N});
         R.push_back(Blk{"rho1", b.rho[1], eb * N});
-        if ((rc = ralloc(R, "mass", &b.mass, N)) || (rc = ralloc(R, "uS", &b.uS, 3 * N)) ||
-            (rc = ralloc(R, "hFi", &b.hFi, 3 * N)) || (rc = ralloc(R, "claim", &b.claim, N)) ||
-            (rc = ralloc(R, "list0", &b.list[0], N)) || (rc = ralloc(R, "list1", &b.list[1], N)) ||
-            (rc = ralloc(R, "listA", &b.listA, N)) || (rc = ralloc(R, "listB", &b.listB, N)) ||
-            (rc = ralloc(R, "mnew", &b.mnew, N)) || (rc = ralloc(R, "state", &b.state, N)) ||
-            (rc = ralloc(R, "ctr", &b.ctr, 1)))
+        if ((rc = ralloc(A, R, "mass", &b.mass, N)) || (rc = ralloc(A, R, "uS", &b.uS, 3 * N)) ||
+            (rc = ralloc(A, R, "hFi", &b.hFi, 3 * N)) || (rc = ralloc(A, R, "claim", &b.claim, N)) ||
+            (rc = ralloc(A, R, "list0", &b.list[0], N)) || (rc = ralloc(A, R, "list1", &b.list[1], N)) ||
+            (rc = ralloc(A, R, "listA", &b.listA, N)) || (rc = ralloc(A, R, "listB", &b.listB, N)) ||
+            (rc = ralloc(A, R, "mnew", &b.mnew, N)) || (rc = ralloc(A, R, "state", &b.state, N)) ||
+            (rc = ralloc(A, R, "ctr", &b.ctr, 1)))
             return rc;
-        if (l->hasSlip() && (rc = ralloc(R, "actPrev", &b.actPrev, N))) return rc;
+        if (l->hasSlip() && (rc = ralloc(A, R, "actPrev", &b.actPrev, N))) return rc;
     }
     l->slotCap = slotCap;
     if (slotCap > 0) {
-        if ((rc = dalloc(&l->cp, slotCap)) || (rc = dalloc(&l->cpf, slotCap)) || (rc = dalloc(&l->boxes, slotCap)) ||
-            (rc = dalloc(&l->segs, (size_t)slotCap * l->segCap)) || (rc = dalloc(&l->segCount, slotCap)))
+        if ((rc = dalloc(A, &l->cp, slotCap)) || (rc = dalloc(A, &l->cpf, slotCap)) || (rc = dalloc(A, &l->boxes, slotCap)) ||
+            (rc = dalloc(A, &l->segs, (size_t)slotCap * l->segCap)) || (rc = dalloc(A, &l->segCount, slotCap)))
             return rc;
         HIPCHK(hipMemset(l->segCount, 0, sizeof(uint32_t) * (size_t)slotCap));
     }
@@ -1064,7 +1111,7 @@ int hyb_lb_init(hyb_lb* l, hyb_dem* d) {  // LB.cpp:190-219
     int rc = lb_alloc(l, d && d->P ? slotCap : 0);
     if (rc) return rc;
     // the curved-wall rule tests the type of the node behind as it was when streamed
-    if (cylinders && l->freeSurface && !l->fsb.actPrev && (rc = ralloc(l->saved, "actPrev", &l->fsb.actPrev, l->N)))
+    if (cylinders && l->freeSurface && !l->fsb.actPrev && (rc = ralloc(l->arena, l->saved, "actPrev", &l->fsb.actPrev, l->N)))
         return rc;
     CylSet cs;
     cs.n = 0;
@@ -1072,8 +1119,9 @@ int hyb_lb_init(hyb_lb* l, hyb_dem* d) {  // LB.cpp:190-219
         cs.n = (int)std::min<size_t>(d->cylinders.size(), 2);
         for (int k = 0; k < cs.n; ++k) cs.c[k] = d->cylinders[k];
         l->cyl = d->cylinders[0];  // the curved-wall distances use the first cylinder (LB.cpp:597)
-        if ((rc = ralloc(l->saved, "curvw", &l->curvw, l->N)) || (rc = ralloc(l->saved, "mac0", &l->macBuf[0], 4 * l->N)) ||
-            (rc = ralloc(l->saved, "mac1", &l->macBuf[1], 4 * l->N)))
+        if ((rc = ralloc(l->arena, l->saved, "curvw", &l->curvw, l->N)) ||
+            (rc = ralloc(l->arena, l->saved, "mac0", &l->macBuf[0], 4 * l->N)) ||
+            (rc = ralloc(l->arena, l->saved, "mac1", &l->macBuf[1], 4 * l->N)))
             return rc;
         HIPCHK(hipMemset(l->macBuf[0], 0, 32 * l->N));
         HIPCHK(hipMemset(l->macBuf[1], 0, 32 * l->N));
@@ -1272,6 +1320,35 @@ int hyb_lb_step(hyb_lb* l, hyb_dem* d) {  // LB.cpp:221-233 fused into one kerne
     return HYB_OK;
 }
 
+// Calls f(i0, i1) for consecutive node ranges whose packed values (`per` bytes a node) fit the handle's view
+// buffer, in order on its stream, and waits at the end. The buffer is kept, grown to what was asked for so far
+// up to VIEW_BYTES: large enough that the copies run at their full rate, small beside the lattice. Where the
+// device has no room for it, smaller ranges do.
+constexpr size_t VIEW_BYTES = (size_t)64 << 20, VIEW_LEAST = (size_t)1 << 16;
+extern "C++" template <class F>
+static int view_chunks(hyb_lb* l, size_t per, F&& f) {
+    const size_t most = std::min(VIEW_BYTES, per * l->N);
+    if (l->viewBytes < most) {
+        HIPCHK(hipStreamSynchronize(l->stream));
+        dfree(l->view);
+        l->viewBytes = 0;
+        size_t want = most;
+        while (hipMalloc(&l->view, want) != hipSuccess) {
+            (void)hipGetLastError();
+            l->view = nullptr;
+            if (want <= VIEW_LEAST) return fail(HYB_E_HIP, "view buffer allocation failed");
+            want /= 2;
+        }
+        l->viewBytes = want;
+    }
+    const size_t chunk = l->viewBytes / per;
+    for (size_t i0 = 0; i0 < l->N; i0 += chunk)
+        if (int rc = f(i0, std::min(l->N, i0 + chunk))) return rc;
+    HIPCHK(hipGetLastError());
+    HIPCHK(hipStreamSynchronize(l->stream));
+    return HYB_OK;
+}
+
 int hyb_lb_set_force_field(hyb_lb* l, const float* F) {
     if (!l || !l->inited) return fail(HYB_E_STATE, "hyb_lb_set_force_field before init");
     HIPCHK(hipStreamSynchronize(l->stream));
@@ -1284,35 +1361,25 @@ int hyb_lb_set_force_field(hyb_lb* l, const float* F) {
         return HYB_OK;
     }
     const size_t N = l->N;
-    std::vector<float> planes(3 * N);
-    for (size_t i = 0; i < N; ++i)
-        for (int k = 0; k < 3; ++k) planes[(size_t)k * N + i] = F[3 * i + k];
     int rc;
     if (!l->ffield && (rc = ralloc(l->saved, "ffield", &l->ffield, 3 * N))) return rc;
-    HIPCHK(hipMemcpy(l->ffield, planes.data(), 12 * N, hipMemcpyHostToDevice));
-    return HYB_OK;
+    return view_chunks(l, 12, [&](size_t i0, size_t i1) -> int {
+        HIPCHK(hipMemcpyAsync(l->view, F + 3 * i0, 12 * (i1 - i0), hipMemcpyHostToDevice, l->stream));
+        launch_fill_force((const float*)l->view, l->ffield, N, i0, i1, l->stream);
+        return HYB_OK;
+    });
 }
 
 int hyb_lb_set_populations(hyb_lb* l, const double* f) {
     if (!l || !f) return fail(HYB_E_ARG, "hyb_lb_set_populations: null argument");
     if (!l->inited || l->steps != 0) return fail(HYB_E_STATE, "populations can only be set before the first step");
     HIPCHK(hipStreamSynchronize(l->stream));
-    const size_t N = l->N, PS = l->planeStride();
-    std::vector<uint32_t> lk(N);
-    HIPCHK(hipMemcpy(lk.data(), l->link, N * 4, hipMemcpyDeviceToHost));
-    if (l->prec == Prec::F64) {
-        std::vector<double> pl(19 * PS, 0.0);
-        for (size_t i = 0; i < N; ++i)
-            if (lk[i] & LINK_ACTIVE)
-                for (int j = 0; j < 19; ++j) pl[(size_t)j * PS + i] = f[i * 19 + j];
-        HIPCHK(hipMemcpy(l->f[l->cur], pl.data(), pl.size() * 8, hipMemcpyHostToDevice));
-    } else {
-        std::vector<float> pl(19 * PS, 0.0f);
-        for (size_t i = 0; i < N; ++i)
-            if (lk[i] & LINK_ACTIVE)
-                for (int j = 0; j < 19; ++j) pl[(size_t)j * PS + i] = (float)(f[i * 19 + j] - wgt(j));
-        HIPCHK(hipMemcpy(l->f[l->cur], pl.data(), pl.size() * 4, hipMemcpyHostToDevice));
-    }
+    const int rc = view_chunks(l, 19 * 8, [&](size_t i0, size_t i1) -> int {
+        HIPCHK(hipMemcpyAsync(l->view, f + 19 * i0, 19 * 8 * (i1 - i0), hipMemcpyHostToDevice, l->stream));
+        launch_fill_pops(l->prec, (const double*)l->view, l->f[l->cur], l->planeStride(), l->link, i0, i1, l->stream);
+        return HYB_OK;
+    });
+    if (rc) return rc;
     l->macValid = false;
     return HYB_OK;
 }
@@ -1329,11 +1396,10 @@ static int adj_check(hyb_lb* l) {
 
 // Releases the checkpoints and the reverse pass's buffers.
 static void adj_free(hyb_lb* l) {
-    for (void* q : l->adjCk) (void)hipFree(q);
-    for (void* q : l->adjSeg) (void)hipFree(q);
+    l->adjArena.release();
     l->adjCk.clear();
     l->adjSeg.clear();
-    dfree(l->adjLam[0]); dfree(l->adjLam[1]); dfree(l->adjGF); dfree(l->adjTP);
+    l->adjLam[0] = l->adjLam[1] = l->adjGF = l->adjTP = nullptr;
     l->adjSteps = -1;
 }
 
@@ -1356,17 +1422,24 @@ int hyb_adj_forward(hyb_lb* l, hyb_dem* d, int32_t steps, int32_t every) {
     const size_t pb = l->popBytes();
     const int M = (steps + every - 1) / every;  // checkpoints of s_0, s_k, ..., s_{(M-1)k}
     const int K = std::min(every, steps);        // states of one interval in the reverse pass
-    auto grab = [&](std::vector<void*>& v, int n) -> int {
+    // Slabs of whole states, up to 256 MiB: thirty-one states of 42 x 37 x 31 nodes fit one (a gradient 20.0 -> 12.2
+    // ms), a state of 128^3 nodes has one of its own. Larger slabs for these made the first gradient of a process
+    // slower (199 ms; slabs of 1 GiB 216, one of 10 GB 360 to 1400, one per state 186) and a repeated one only 5 %
+    // faster.
+    const size_t need = 8 * adj_tau_slots(l->params()) + 24 * l->N + pb * (size_t)(M + K + 2) + ARENA_ALIGN * (size_t)(M + K + 4);
+    const size_t one = (pb + ARENA_ALIGN - 1) / ARENA_ALIGN * ARENA_ALIGN;
+    l->adjArena.slab = std::min(need, one * std::max<size_t>(1, ((size_t)256 << 20) / one));
+    const auto grab = [&](std::vector<void*>& v, int n) -> int {
         for (int m = 0; m < n; ++m) {
             void* q = nullptr;
-            if (hipMalloc(&q, pb) != hipSuccess) return fail(HYB_E_HIP, "adjoint buffer allocation failed");
+            if (int rc2 = l->adjArena.take(&q, pb)) return rc2;
             v.push_back(q);
         }
         return HYB_OK;
     };
-    if ((rc = grab(l->adjCk, M)) || (rc = grab(l->adjSeg, K)) || (rc = dalloc(&l->adjLam[0], pb / 8)) ||
-        (rc = dalloc(&l->adjLam[1], pb / 8)) || (rc = dalloc(&l->adjGF, 3 * l->N)) ||
-        (rc = dalloc(&l->adjTP, adj_tau_slots(l->params())))) {
+    if ((rc = grab(l->adjCk, M)) || (rc = grab(l->adjSeg, K)) || (rc = dalloc(l->adjArena, &l->adjLam[0], pb / 8)) ||
+        (rc = dalloc(l->adjArena, &l->adjLam[1], pb / 8)) || (rc = dalloc(l->adjArena, &l->adjGF, 3 * l->N)) ||
+        (rc = dalloc(l->adjArena, &l->adjTP, adj_tau_slots(l->params())))) {
         adj_free(l);
         return rc;
     }
@@ -1465,23 +1538,15 @@ int hyb_lb_destroy(hyb_lb* l) {
     if (!l) return HYB_OK;
     if (l->stream) (void)hipStreamSynchronize(l->stream);
     for (auto& ev : l->evs) (void)hipEventDestroy(ev);
-    if (l->f[0]) (void)hipFree(l->f[0]);
-    if (l->f[1]) (void)hipFree(l->f[1]);
     if (l->scratch) (void)hipFree(l->scratch);
-    dfree(l->type); dfree(l->link); dfree(l->slipw); dfree(l->solid); dfree(l->visc); dfree(l->mac); dfree(l->maxXYZ);
-    dfree(l->curvw); dfree(l->macBuf[0]); dfree(l->macBuf[1]);
-    dfree(l->dcount); dfree(l->cp); dfree(l->cpf); dfree(l->boxes); dfree(l->nslots); dfree(l->segs);
-    dfree(l->segCount);
+    if (l->view) (void)hipFree(l->view);
+    dfree(l->mac);
     adj_free(l);
     for (hipEvent_t ev : l->adjEv)
         if (ev) (void)hipEventDestroy(ev);
     if (l->ffield) (void)hipFree(l->ffield);
     errword_free(l->err);
-    FSBuffers& b = l->fsb;
-    if (b.rho[0]) (void)hipFree(b.rho[0]);
-    if (b.rho[1]) (void)hipFree(b.rho[1]);
-    dfree(b.mass); dfree(b.uS); dfree(b.hFi); dfree(b.claim); dfree(b.list[0]); dfree(b.list[1]); dfree(b.listA);
-    dfree(b.listB); dfree(b.mnew); dfree(b.state); dfree(b.ctr); dfree(b.actPrev);
+    l->arena.release();
     delete l;
     return HYB_OK;
 }
@@ -1621,30 +1686,35 @@ int hyb_lb_get(hyb_lb* l, const char* cname, void* host, size_t cap, size_t* nee
     const std::string name(cname);
     const size_t N = l->N;
     const LBKParams p = l->params();
-    std::vector<uint32_t> lk(N);
-    HIPCHK(hipMemcpy(lk.data(), l->link, N * 4, hipMemcpyDeviceToHost));
+    // a view of `per` bytes a node: launch packs nodes [i0, i1) into the view buffer
+    const auto packed = [&](size_t per, auto&& launch) -> int {
+        return view_chunks(l, per, [&](size_t i0, size_t i1) -> int {
+            launch(i0, i1);
+            HIPCHK(hipMemcpyAsync((char*)host + per * i0, l->view, per * (i1 - i0), hipMemcpyDeviceToHost, l->stream));
+            return HYB_OK;
+        });
+    };
+    const auto wanted = [&](size_t bytes) {  // whether the values are asked for, not only their size
+        if (need) *need = bytes;
+        return host && cap >= bytes;
+    };
     if (name == "types") {
-        std::vector<uint8_t> t(N);
-        HIPCHK(hipMemcpy(t.data(), l->type, N, hipMemcpyDeviceToHost));
-        return put(t.data(), N, host, cap, need);
+        if (wanted(N)) {
+            HIPCHK(hipMemcpyAsync(host, l->type, N, hipMemcpyDeviceToHost, l->stream));
+            HIPCHK(hipStreamSynchronize(l->stream));
+        }
+        return HYB_OK;
     }
     if (name == "pflag" || name == "solidIndex") {  // particle nodes are active nodes (LB.cpp:475-495)
-        std::vector<uint32_t> so(N), lw(N);
-        HIPCHK(hipMemcpy(so.data(), l->solid, N * 4, hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(lw.data(), l->link, N * 4, hipMemcpyDeviceToHost));
-        for (size_t i = 0; i < N; ++i)
-            so[i] = ((lw[i] & LINK_ACTIVE) && (so[i] >> SOLID_SLOT_BITS) == l->ctag) ? (so[i] & SOLID_SLOT_MASK) : 0u;
-        if (name == "pflag") {
-            std::vector<uint8_t> pf(N);
-            for (size_t i = 0; i < N; ++i) pf[i] = so[i] ? 1 : 0;
-            return put(pf.data(), N, host, cap, need);
-        }
-        for (size_t i = 0; i < N; ++i) so[i] = so[i] ? so[i] - 1 : 0xFFFFFFFFu;
-        return put(so.data(), N * 4, host, cap, need);
+        const bool index = name == "solidIndex";
+        const size_t per = index ? 4 : 1;
+        if (!wanted(N * per)) return HYB_OK;
+        return packed(per, [&](size_t i0, size_t i1) {
+            launch_view_owner(l->solid, l->link, l->ctag, index, l->view, i0, i1, l->stream);
+        });
     }
     if (name == "f") {
-        if (need) *need = N * 19 * 8;
-        if (!host || cap < N * 19 * 8) return HYB_OK;
+        if (!wanted(N * 19 * 8)) return HYB_OK;
         const void* src = l->f[l->cur];
         if (l->steps > 0) {
             if (!l->scratch) HIPCHK(hipMalloc(&l->scratch, l->popBytes()));
@@ -1652,63 +1722,47 @@ int hyb_lb_get(hyb_lb* l, const char* cname, void* host, size_t cap, size_t* nee
                 launch_fs_stream_view(l->prec, l->f[l->cur], l->scratch, l->type, l->link, l->fsb.uS, p, l->stream);
             else
                 launch_lb_stream(l->prec, l->f[l->cur], l->scratch, l->link, p, l->stream);
-            HIPCHK(hipGetLastError());
-            HIPCHK(hipStreamSynchronize(l->stream));
             src = l->scratch;
         }
-        double* out = (double*)host;
-        const size_t PS = l->planeStride();
-        if (l->prec == Prec::F64) {
-            std::vector<double> f(19 * PS);
-            HIPCHK(hipMemcpy(f.data(), src, 19 * PS * 8, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < N; ++i)
-                for (int j = 0; j < 19; ++j) out[i * 19 + j] = (lk[i] & LINK_ACTIVE) ? f[(size_t)j * PS + i] : NAN;
-        } else {
-            std::vector<float> f(19 * PS);
-            HIPCHK(hipMemcpy(f.data(), src, 19 * PS * 4, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < N; ++i)
-                for (int j = 0; j < 19; ++j)
-                    out[i * 19 + j] = (lk[i] & LINK_ACTIVE) ? (double)f[(size_t)j * PS + i] + wgt(j) : NAN;
-        }
-        return HYB_OK;
+        return packed(19 * 8, [&](size_t i0, size_t i1) {
+            launch_view_pops(l->prec, src, l->planeStride(), l->link, (double*)l->view, i0, i1, l->stream);
+        });
     }
     if (name == "n" && l->freeSurface) {
-        if (need) *need = N * 8;
-        if (!host || cap < N * 8) return HYB_OK;
-        std::vector<double> r;
-        int rc = fs_density(l, l->rhoCur, r);
-        if (rc) return rc;
-        double* out = (double*)host;
-        for (size_t i = 0; i < N; ++i) out[i] = (lk[i] & LINK_ACTIVE) ? r[i] : NAN;
-        return HYB_OK;
+        if (!wanted(N * 8)) return HYB_OK;
+        return packed(8, [&](size_t i0, size_t i1) {
+            launch_view_scalar(false, nullptr, 0.0, l->fsb.rho[l->rhoCur], l->prec, 0.0, l->link, (double*)l->view, i0, i1,
+                               l->stream);
+        });
     }
     if (name == "n" || name == "u" || name == "hydroForce") {
         const size_t w = name == "n" ? 1 : 3;
-        if (need) *need = N * w * 8;
-        if (!host || cap < N * w * 8) return HYB_OK;
-        int rc = ensure_mac(l, l->dem);
-        if (rc) return rc;
-        std::vector<double> m(7 * N);
-        HIPCHK(hipMemcpy(m.data(), l->mac, 7 * N * 8, hipMemcpyDeviceToHost));
-        double* out = (double*)host;
-        const size_t off = name == "n" ? 0 : (name == "u" ? 1 : 4);
-        for (size_t i = 0; i < N; ++i)
-            for (size_t k = 0; k < w; ++k) out[i * w + k] = (lk[i] & LINK_ACTIVE) ? m[(off + k) * N + i] : NAN;
-        return HYB_OK;
+        if (!wanted(N * w * 8)) return HYB_OK;
+        if (int rc = ensure_mac(l, l->dem)) return rc;
+        const double* planes = l->mac + (name == "n" ? 0 : (name == "u" ? 1 : 4)) * N;
+        return packed(w * 8, [&](size_t i0, size_t i1) {
+            launch_view_planes(planes, N, (int)w, l->link, (double*)l->view, i0, i1, l->stream);
+        });
     }
     if (name == "visc" || name == "mass") {
-        std::vector<double> v(N, NAN);
-        if (name == "visc") {
-            if (l->visc) HIPCHK(hipMemcpy(v.data(), l->visc, N * 8, hipMemcpyDeviceToHost));
-            for (size_t i = 0; i < N; ++i) v[i] = (lk[i] & LINK_ACTIVE) ? (l->visc ? v[i] : l->initDynVisc) : NAN;
-        } else {
-            int rc = mass_view(l, lk, v);
-            if (rc) return rc;
-        }
-        return put(v.data(), N * 8, host, cap, need);
+        if (!wanted(N * 8)) return HYB_OK;
+        return packed(8, [&](size_t i0, size_t i1) {
+            if (name == "visc") {
+                launch_view_scalar(false, nullptr, 0.0, l->visc, Prec::F64, l->initDynVisc, l->link, (double*)l->view, i0, i1,
+                                   l->stream);
+            } else {  // the cases of mass_view
+                const bool tracked = l->freeSurface && l->fsSteps > 0;
+                launch_view_scalar(true, l->freeSurface ? l->fsb.mass : nullptr, 0.5 * l->initDensity,
+                                   tracked ? l->fsb.rho[l->fluidMassBuf] : nullptr, l->prec, l->initDensity, l->link,
+                                   (double*)l->view, i0, i1, l->stream);
+            }
+        });
     }
     if (name == "totalMass") return put(&l->totalMass, 8, host, cap, need);
     if (name == "fluidMass") {  // IO::totFluidMass (IO.cpp:987-999), summed in node order
+        if (!wanted(8)) return HYB_OK;
+        std::vector<uint32_t> lk(N);
+        HIPCHK(hipMemcpy(lk.data(), l->link, N * 4, hipMemcpyDeviceToHost));
         std::vector<double> v(N, NAN);
         int rc = mass_view(l, lk, v);
         if (rc) return rc;
@@ -1871,12 +1925,31 @@ int hyb_dem_get(hyb_dem* d, const char* cname, void* host, size_t cap, size_t* n
     HIPCHK(hipStreamSynchronize(d->stream));
     const std::string name(cname);
     const int P = d->P, NE = d->E;
+    if (int rc = dem_pending(d)) return rc;
+    const auto wanted = [&](size_t bytes) {  // whether the values are asked for, not only their size
+        if (need) *need = bytes;
+        return host && cap >= bytes && bytes;
+    };
+    // rows of `count` consecutive element fields, packed on the device
+    const auto rows = [&](int first, int count) -> int {
+        const size_t bytes = sizeof(double) * (size_t)NE * count;
+        if (!wanted(bytes)) return HYB_OK;
+        launch_view_rows(d->b.el, NE, first, count, d->view, d->stream);
+        HIPCHK(hipGetLastError());
+        HIPCHK(hipMemcpyAsync(host, d->view, bytes, hipMemcpyDeviceToHost, d->stream));
+        HIPCHK(hipStreamSynchronize(d->stream));
+        return HYB_OK;
+    };
+    // at step end the predicted copies equal the corrected ones (elmt.cpp:190-224)
+    if (name == "e_x" || name == "e_xp") return rows(EF_X, 18);
+    if (name == "e_w" || name == "e_wp") return rows(EF_W, 18);
+    if (name == "e_q" || name == "e_qp") return rows(EF_Q, 24);
+    if (name == "e_forces") return rows(EF_FH, 21);
     DEMState st;
     std::memset(&st, 0, sizeof(st));
     if (P) HIPCHK(hipMemcpy(&st, d->b.st, sizeof(st), hipMemcpyDeviceToHost));
-    if (int rc = dem_pending(d)) return rc;
     std::vector<double> el;
-    if (P) {
+    if (P && (name == "e_misc" || name == "p_data")) {
         el.resize((size_t)EF_COUNT * NE);
         HIPCHK(hipMemcpy(el.data(), d->b.el, el.size() * 8, hipMemcpyDeviceToHost));
     }
@@ -1884,9 +1957,11 @@ int hyb_dem_get(hyb_dem* d, const char* cname, void* host, size_t cap, size_t* n
     std::vector<double> v;
     std::vector<uint32_t> u;
     const int G = P ? st.nGhost : 0;
-    std::vector<uint32_t> gi(G);
-    std::vector<double> gv(3 * (size_t)G);
-    if (G) {
+    std::vector<uint32_t> gi;
+    std::vector<double> gv;
+    if (G && (name == "p_data" || name == "p_idx" || name == "ghostIndex" || name == "ghostVec")) {
+        gi.resize(G);
+        gv.resize(3 * (size_t)G);
         HIPCHK(hipMemcpy(gi.data(), d->b.ghostIndex, 4 * (size_t)G, hipMemcpyDeviceToHost));
         HIPCHK(hipMemcpy(gv.data(), d->b.ghostVec, 24 * (size_t)G, hipMemcpyDeviceToHost));
     }
@@ -1967,23 +2042,6 @@ int hyb_dem_get(hyb_dem* d, const char* cname, void* host, size_t cap, size_t* n
             HIPCHK(hipStreamSynchronize(d->stream));
         }
         return put(e6, sizeof(e6), host, cap, need);
-    }
-    if (name == "e_x" || name == "e_xp" || name == "e_w" || name == "e_wp") {
-        // at step end the predicted copies equal the corrected ones (elmt.cpp:190-224)
-        const int base = (name == "e_x" || name == "e_xp") ? EF_X : EF_W;
-        for (int e = 0; e < NE; ++e)
-            for (int k = 0; k < 18; ++k) v.push_back(at(base + k, e));
-        return put(v.data(), v.size() * 8, host, cap, need);
-    }
-    if (name == "e_q" || name == "e_qp") {
-        for (int e = 0; e < NE; ++e)
-            for (int k = 0; k < 24; ++k) v.push_back(at(EF_Q + k, e));
-        return put(v.data(), v.size() * 8, host, cap, need);
-    }
-    if (name == "e_forces") {
-        for (int e = 0; e < NE; ++e)
-            for (int k = 0; k < 21; ++k) v.push_back(at(EF_FH + k, e));
-        return put(v.data(), v.size() * 8, host, cap, need);
     }
     if (name == "e_misc") {
         for (int e = 0; e < NE; ++e) {
