@@ -26,7 +26,7 @@ namespace hyb {
 
 namespace {
 
-constexpr int ABX = 256;
+constexpr int ABX = ROW_BLOCK;
 // at least this many workgroups per CU: caps the registers so that several
 // wavefronts per SIMD hide the latency of the 38 neighbour loads
 #ifndef ADJ_MIN_BLOCKS
@@ -39,24 +39,17 @@ constexpr int ABX = 256;
 #define ADJ_HOIST 1
 #endif
 // non-temporal loads of the state and adjoint populations and stores of the
-// new adjoint populations (each is touched once per step)
-#ifndef ADJ_NT
-#define ADJ_NT 1
-#endif
+// new adjoint populations (each is touched once per step) where the lines are
+// whole, as in the forward step
 
+template <bool MERGE>
 __device__ __forceinline__ double ld_nt(const double* p) {
-#if ADJ_NT
-    return __builtin_nontemporal_load(p);
-#else
-    return *p;
-#endif
+    return MERGE ? *p : __builtin_nontemporal_load(p);
 }
+template <bool MERGE>
 __device__ __forceinline__ void st_nt(double* p, double v) {
-#if ADJ_NT
-    __builtin_nontemporal_store(v, p);
-#else
-    *p = v;
-#endif
+    if (MERGE) *p = v;
+    else __builtin_nontemporal_store(v, p);
 }
 
 // Neighbour index along direction j (periodic rewiring) as a 32-bit offset.
@@ -67,31 +60,36 @@ __device__ __forceinline__ uint32_t nb32(const Nb3& nx, const Nb3& ny, const Nb3
 // The vector-Jacobian product runs over the 9 direction pairs (i, opp i = i + 1)
 // and the rest direction, using c_opp = -c_i and w_opp = w_i, so that only the
 // incoming populations and the adjoint populations stay in registers.
-template <int COLL>
+template <int COLL, bool MERGE>
 __global__ void __launch_bounds__(ABX, ADJ_MIN_BLOCKS)
     k_adj_step(const double* __restrict__ sPrev, const double* __restrict__ lamNext, double* __restrict__ lamOut,
                const uint32_t* __restrict__ link, const uint32_t* __restrict__ solid, const CoupleRec* __restrict__ cp,
                double* __restrict__ gradF, double* __restrict__ tauPart, LBKParams p, int pullFwd) {
 #pragma clang fp contract(off)
     __shared__ double red[ABX / 64];
-    const int x = blockIdx.x * ABX + threadIdx.x, y = blockIdx.y, z = blockIdx.z;
+    Coord c;
+    const bool inRange = lane_coord<MERGE>(p, c);
+    const int x = c.x, y = c.y, z = c.z;
     const size_t N = (size_t)p.X * p.Y * p.Z;
     double tauAcc = 0.0;
-    const bool inRange = x < p.X;
-    const uint32_t self = inRange ? (uint32_t)x + (uint32_t)p.X * ((uint32_t)y + (uint32_t)p.Y * (uint32_t)z) : 0u;
+    const uint32_t self = inRange ? (uint32_t)c.idx : 0u;
     const uint32_t lw = inRange ? link[self] : 0u;
-    if (lw & LINK_ACTIVE) {
+    const bool act = (lw & LINK_ACTIVE) != 0u;
+    const bool fill = inRange && fills_line<double>(act);
+    double m[19], nbar = 0.0;
+    V3 jbar;
+    if (act) {
         const Nb3 nx = nb3(x, p.X, p.per[0]), ny = nb3(y, p.Y, p.per[1]), nz = nb3(z, p.Z, p.per[2]);
         const uint32_t sX = (uint32_t)p.X, sXY = (uint32_t)p.X * (uint32_t)p.Y;
         // g_t: populations entering this node's collision; f_i arrives from the
         // neighbour in direction opp(i) (or bounces back from a static wall there)
-        double g[19], m[19];
+        double g[19];
         if (pullFwd) {
             // the 19 loads back to back; a static-wall neighbour's index is valid
             // memory and its value is replaced by the bounce-back below
 #pragma unroll
             for (int i = 0; i < 19; ++i)
-                g[i] = ld_nt(&sPrev[(size_t)i * p.PS + (i == 0 ? self : nb32(nx, ny, nz, sX, sXY, opp(i)))]);
+                g[i] = ld_nt<MERGE>(&sPrev[(size_t)i * p.PS + (i == 0 ? self : nb32(nx, ny, nz, sX, sXY, opp(i)))]);
             if (lw & LINK_WALLS) {
 #pragma unroll
                 for (int i = 1; i < 19; ++i)
@@ -105,7 +103,7 @@ __global__ void __launch_bounds__(ABX, ADJ_MIN_BLOCKS)
         const auto load_mu = [&]() {
 #pragma unroll
             for (int j = 0; j < 19; ++j)
-                m[j] = ld_nt(&lamNext[(size_t)j * p.PS + (j == 0 ? self : nb32(nx, ny, nz, sX, sXY, j))]);
+                m[j] = ld_nt<MERGE>(&lamNext[(size_t)j * p.PS + (j == 0 ? self : nb32(nx, ny, nz, sX, sXY, j))]);
             if (lw & LINK_WALLS) {
 #pragma unroll
                 for (int j = 1; j < 19; ++j)
@@ -169,7 +167,7 @@ __global__ void __launch_bounds__(ABX, ADJ_MIN_BLOCKS)
         asm volatile("" : "+v"(usx), "+v"(usy), "+v"(usz), "+v"(Tx), "+v"(Ty), "+v"(Tz));
         if (!ADJ_HOIST) load_mu();
         // ---- reverse
-        double nbar = 0.0, qbar = 0.0, rbar = 0.0, omPbar = 0.0, omMbar = 0.0;
+        double qbar = 0.0, rbar = 0.0, omPbar = 0.0, omMbar = 0.0;
         V3 usbar, Tbar;
         {  // rest direction: c = 0, so a = b = 0, no odd part
             const double w = wgt(0), mi = m[0];
@@ -229,11 +227,16 @@ __global__ void __launch_bounds__(ABX, ADJ_MIN_BLOCKS)
             nbar += (pm / (n * n)) * Tbar.dot(dv);
         }
         // u = j / n
-        const V3 jbar = ubar / n;
+        jbar = ubar / n;
         nbar += -ubar.dot(u) / n;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 19; ++i) m[i] = 0.0;
+    }
+    if (act || fill) {
 #pragma unroll
         for (int i = 0; i < 19; ++i)
-            st_nt(&lamOut[(size_t)i * p.PS + self],
+            st_nt<MERGE>(&lamOut[(size_t)i * p.PS + self],
                   m[i] + nbar + (double)cx(i) * jbar.x + (double)cy(i) * jbar.y + (double)cz(i) * jbar.z);
     }
     // workgroup sum of the tau gradient in a fixed order
@@ -242,7 +245,7 @@ __global__ void __launch_bounds__(ABX, ADJ_MIN_BLOCKS)
     __syncthreads();
     if (threadIdx.x == 0) {
         double s = 0.0;
-        for (int w = 0; w < ABX / 64; ++w) s += red[w];
+        for (int w = 0; w < (int)blockDim.x / 64; ++w) s += red[w];
         const size_t slot = (size_t)blockIdx.x + (size_t)gridDim.x * ((size_t)blockIdx.y + (size_t)gridDim.y * blockIdx.z);
         tauPart[slot] += s;
     }
@@ -273,18 +276,26 @@ void launch_planes_to_nodes(const double* src, double* dst, const uint32_t* link
     k_planes_to_nodes<<<4096, 256, 0, s>>>(src, dst, link, N, PS, Q);
 }
 
-size_t adj_tau_slots(const LBKParams& p) { return (size_t)((p.X + ABX - 1) / ABX) * p.Y * p.Z; }
+size_t adj_tau_slots(const LBKParams& p) {
+    const dim3 g = merge_map(p, Prec::F64) ? merge_grid(p) : row_grid(p);
+    return (size_t)g.x * g.y * g.z;
+}
 
 void launch_adj_step(int collision, const double* sPrev, const double* lamNext, double* lamOut, const uint32_t* link,
                      const uint32_t* solid, const CoupleRec* cp, double* gradF, double* tauPart, bool pullFwd,
                      const LBKParams& p, hipStream_t s) {
-    const dim3 g((p.X + ABX - 1) / ABX, p.Y, p.Z), b(ABX, 1, 1);
-    if (collision == HYB_COLLISION_TRT)
-        k_adj_step<HYB_COLLISION_TRT><<<g, b, 0, s>>>(sPrev, lamNext, lamOut, link, solid, cp, gradF, tauPart, p,
-                                                      pullFwd ? 1 : 0);
-    else
-        k_adj_step<HYB_COLLISION_BGK><<<g, b, 0, s>>>(sPrev, lamNext, lamOut, link, solid, cp, gradF, tauPart, p,
-                                                      pullFwd ? 1 : 0);
+    const bool merge = merge_map(p, Prec::F64);
+    const dim3 g = merge ? merge_grid(p) : row_grid(p), b = row_block(p);
+#define HYB_ADJ_CASE(CO, MERGE)                                                                                      \
+    if (collision == CO && merge == MERGE) {                                                                         \
+        k_adj_step<CO, MERGE><<<g, b, 0, s>>>(sPrev, lamNext, lamOut, link, solid, cp, gradF, tauPart, p,           \
+                                             pullFwd ? 1 : 0);                                                     \
+        return;                                                                                                    \
+    }
+    HYB_ADJ_CASE(HYB_COLLISION_BGK, false)
+    HYB_ADJ_CASE(HYB_COLLISION_BGK, true)
+    HYB_ADJ_CASE(HYB_COLLISION_TRT, false)
+    HYB_ADJ_CASE(HYB_COLLISION_TRT, true)
 }
 
 }  // namespace hyb

@@ -20,6 +20,7 @@
 #include "dem_kernels.h"
 #include "fs_kernels.h"
 #include "hybird_amd.h"
+#include "lattice.h"
 #include "lb_kernels.h"
 #include "view_kernels.h"
 
@@ -366,6 +367,9 @@ struct hyb_lb {
         p.viscw = varVisc() ? visc : nullptr;
         p.cyl = cyl;
         p.herr = err.dev;
+        const dim3 g = row_grid(p);
+        p.invRows = inverse_of((uint64_t)g.x * g.y);
+        p.invChunks = inverse_of(g.y);
         return p;
     }
     // planes are padded so that successive planes do not start on the same

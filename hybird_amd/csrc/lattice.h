@@ -27,6 +27,90 @@ __device__ __forceinline__ Coord coord_of(const LBKParams& p, size_t idx) {
     return c;
 }
 
+// ---- node-to-lane map of the kernels that visit every node
+// A wavefront takes 64 consecutive x nodes of one row, a workgroup up to four wavefronts: of four rows where X <= 64,
+// of two where X <= 128, else of one row, whose wavefronts are spread evenly over its workgroups. (256 lanes on one
+// row left three of four wavefronts empty at X = 64 and every other workgroup of X = 384 with 128 nodes of padding.)
+// y runs fastest over the workgroups, which the hardware deals to the eight XCDs in turn: with x fastest a liquid
+// that fills the low x of an X = 384 lattice put all its work on every second XCD.
+constexpr int ROW_BLOCK = 256;  // most lanes of a workgroup
+__host__ __device__ __forceinline__ int row_shift(int X) { return X <= 64 ? 2 : (X <= 128 ? 1 : 0); }
+inline int row_chunks(const LBKParams& p) { return (p.X + ROW_BLOCK - 1) / ROW_BLOCK; }
+inline dim3 row_block(const LBKParams& p) {
+    const int waves = (p.X + 63) / 64, n = row_chunks(p);
+    return dim3(row_shift(p.X) ? ROW_BLOCK : 64 * ((waves + n - 1) / n), 1, 1);
+}
+inline dim3 row_grid(const LBKParams& p) {
+    const int rows = 1 << row_shift(p.X);
+    return dim3((p.Y + rows - 1) / rows, row_chunks(p), p.Z);
+}
+// The node of this lane (false: none). The wavefront's row is made uniform so that row offsets stay in scalar registers.
+__device__ __forceinline__ bool row_coord(const LBKParams& p, Coord& c) {
+    const int rl = row_shift(p.X), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const int chunk = (int)blockIdx.y * ((int)blockDim.x >> 6);  // blockIdx.y is 0 where a workgroup has several rows
+    c.x = 64 * (chunk + (wave & ((4 >> rl) - 1))) + ((int)threadIdx.x & 63);
+    c.y = ((int)blockIdx.x << rl) + (wave >> (2 - rl));
+    c.z = (int)blockIdx.z;
+    if (c.x >= p.X || c.y >= p.Y) return false;
+    c.idx = (size_t)c.x + (size_t)p.X * ((size_t)c.y + (size_t)p.Y * (size_t)c.z);
+    return true;
+}
+
+// Rows that don't end on a 128-byte line share one with the next row, written in part by two workgroups. There the
+// XCDs take MERGE_RUN consecutive workgroups at a time instead of one, x fastest, and the populations are not streamed
+// past the L2, which then completes the lines. us per 10^6 nodes of X x 150 x 150, row map against this one: FP32
+// X = 40 48.2 / 34.9, 100 43.5 / 37.3, 150 50.0 / 36.2, 257 52.5 / 43.6; FP64 X = 40 77.4 / 67.4, 150 78.2 / 64.0, 300
+// 70.1 / 66.5. Where the rows do end on lines the row map is ahead: FP32 X = 96 30.3 / 33.4, 160 29.5 / 31.7; FP64
+// X = 80 58.7 / 62.3, 240 56.5 / 58.2. Runs of 4 and of 64 workgroups were within 2 %; streaming loads or stores
+// alone lost (X = 150: 34.9 and 42.0, FP64 67.7 and 73.0). 64 consecutive nodes of the whole lattice per wavefront
+// (32.8, FP64 58.8) would cut the run sums below elsewhere and change their rounding.
+constexpr int MERGE_RUN = 16, XCDS = 8;
+inline bool merge_map(const LBKParams& p, Prec prec) {
+    return (size_t)p.X * (prec == Prec::F64 ? 8 : 4) % 128 != 0;
+}
+inline dim3 merge_grid(const LBKParams& p) {
+    const dim3 g = row_grid(p);
+    const size_t n = (size_t)g.x * g.y * g.z, per = (size_t)MERGE_RUN * XCDS;
+    return dim3((unsigned)((n + per - 1) / per * per), 1, 1);
+}
+// n / d for inv = ceil(2^64 / d), 0 for d = 1: the error n (inv d - 2^64) / (d 2^64) is below 1 / d for 32-bit n, d.
+inline uint64_t inverse_of(uint64_t d) { return d == 1 ? 0ull : ~0ull / d + 1ull; }
+__device__ __forceinline__ uint32_t div_by(uint32_t n, uint64_t inv) {
+    return inv ? (uint32_t)__umul64hi((uint64_t)n, inv) : n;
+}
+__device__ __forceinline__ bool merge_coord(const LBKParams& p, Coord& c) {
+    const int rl = row_shift(p.X), wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+    const uint32_t b = blockIdx.x, j = b / XCDS;
+    const uint32_t item = ((j / MERGE_RUN) * XCDS + b % XCDS) * MERGE_RUN + j % MERGE_RUN;
+    const uint32_t chunks = (uint32_t)(p.X + ROW_BLOCK - 1) / ROW_BLOCK, groups = (uint32_t)(p.Y + (1 << rl) - 1) >> rl;
+    const uint32_t z = div_by(item, p.invRows), r = item - z * (groups * chunks);
+    const uint32_t y = div_by(r, p.invChunks), chunk = (r - y * chunks) * (blockDim.x >> 6);
+    c.x = 64 * ((int)chunk + (wave & ((4 >> rl) - 1))) + ((int)threadIdx.x & 63);
+    c.y = ((int)y << rl) + (wave >> (2 - rl));
+    c.z = (int)z;
+    if (c.x >= p.X || c.y >= p.Y || c.z >= p.Z) return false;
+    c.idx = (size_t)c.x + (size_t)p.X * ((size_t)c.y + (size_t)p.Y * (size_t)c.z);
+    return true;
+}
+template <bool MERGE>
+__device__ __forceinline__ bool lane_coord(const LBKParams& p, Coord& c) {
+    return MERGE ? merge_coord(p, c) : row_coord(p, c);
+}
+
+// Whether an inactive lane stores populations with the active ones of its wavefront: where the 128-byte line of its
+// node holds an active node, so that the line is written whole. Nothing reads an inactive node's populations. A line
+// written in part costs the memory a read as well: the ghost layers at both ends of a row alone made the FP32 step of
+// 256^3 nodes 562 us instead of 465, of 64 x 150 x 150 nodes 79 instead of 47. The stores of both kinds of lanes
+// are the same instructions (stores of their own for the inactive lanes made FP64 steps 13 to 40 % slower than none).
+// All lanes of the wavefront that hold a node take part.
+template <typename T>
+__device__ __forceinline__ bool fills_line(bool act) {
+    constexpr int LINE = 128 / (int)sizeof(T);
+    const unsigned long long m = __ballot(act);
+    const int lane = (int)(threadIdx.x & 63u);
+    return !act && ((m >> (lane & ~(LINE - 1))) & (~0ull >> (64 - LINE))) != 0ull;
+}
+
 // Neighbour coordinates x-1, x, x+1 along one axis for an interior node, with the
 // periodic rewiring of LB.cpp:437-472 (layers 0 and X-1 are ghosts, period X-2).
 struct Nb3 {

@@ -28,52 +28,18 @@ namespace {
 // no curved walls) are compiled for 8 (FP32) and 5 (FP64) wavefronts per SIMD,
 // which they reach without spilling (more loads in flight for a bandwidth-bound
 // kernel); the others keep the compiler's register choice.
-// Workgroup tile of the lattice kernels: a full 256-node x-row per workgroup
-// keeps the +-1 x-shifted loads of a row inside one workgroup's cache.
-#ifndef HYB_LB_BX
-#define HYB_LB_BX 256
-#endif
-#ifndef HYB_LB_BY
-#define HYB_LB_BY 1
-#endif
-#ifndef HYB_LB_NT
-#define HYB_LB_NT 1
-#endif
-constexpr int BX = HYB_LB_BX;
-
-constexpr int BY = HYB_LB_BY;
-
-#ifndef HYB_LB_NTLOAD
-#define HYB_LB_NTLOAD 1
-#endif
 
 
-// Population stores and loads: optionally non-temporal (every population is
-// written once and read once per step, so neither benefits from caching).
-template <typename T>
+// Population stores and loads: non-temporal where the lines are whole (every population is written once and read
+// once per step, so neither benefits from caching), plain where rows share lines (MERGE, see merge_coord).
+template <bool MERGE, typename T>
 __device__ __forceinline__ void st_pop(T* p, T v) {
-#if HYB_LB_NT
-    __builtin_nontemporal_store(v, p);
-#else
-    *p = v;
-#endif
+    if (MERGE) *p = v;
+    else __builtin_nontemporal_store(v, p);
 }
-template <typename T>
+template <bool MERGE, typename T>
 __device__ __forceinline__ T ld_pop(const T* p) {
-#if HYB_LB_NTLOAD
-    return __builtin_nontemporal_load(p);
-#else
-    return *p;
-#endif
-}
-
-__device__ __forceinline__ bool node_coord(const LBKParams& p, Coord& c) {
-    c.x = blockIdx.x * BX + threadIdx.x;
-    c.y = blockIdx.y * BY + threadIdx.y;
-    c.z = blockIdx.z;
-    if (c.x >= p.X || c.y >= p.Y) return false;
-    c.idx = (size_t)c.x + (size_t)p.X * ((size_t)c.y + (size_t)p.Y * (size_t)c.z);
-    return true;
+    return MERGE ? *p : __builtin_nontemporal_load(p);
 }
 
 // Whether node n was active when the reference streamed the populations this
@@ -91,11 +57,11 @@ __device__ __forceinline__ bool active_at_stream(const LBKParams& p, size_t n) {
 // walls bounce back the node's own f_opp(i) instead; they only occur next to
 // walls, so that fix-up runs as a separate, rarely taken branch and the common
 // path issues its 19 loads back to back.
-template <typename T, bool CURVED>
+template <typename T, bool CURVED, bool MERGE>
 __device__ __forceinline__ void wall_fixup(const T* __restrict__ fin, size_t PS, const LBKParams& p, const Coord& c,
                                            uint32_t lw, T f[19]);
 
-template <typename T, bool CURVED = false>
+template <typename T, bool CURVED, bool MERGE>
 __device__ __forceinline__ void pull19(const T* __restrict__ fin, size_t PS, const LBKParams& p, const Coord& c,
                                        uint32_t lw, T f[19]) {
     const Nb3 nx = nb3(c.x, p.X, p.per[0]);
@@ -108,15 +74,15 @@ __device__ __forceinline__ void pull19(const T* __restrict__ fin, size_t PS, con
         const int j = opp(i);
         const uint32_t nb = (uint32_t)pick(nx, cx(j)) + sX * (uint32_t)pick(ny, cy(j)) + sXY * (uint32_t)pick(nz, cz(j));
         // a wall neighbour's index is valid memory; its value is replaced below
-        f[i] = ld_pop(&fin[(size_t)i * PS + (i == 0 ? self : nb)]);
+        f[i] = ld_pop<MERGE>(&fin[(size_t)i * PS + (i == 0 ? self : nb)]);
     }
-    wall_fixup<T, CURVED>(fin, PS, p, c, lw, f);
+    wall_fixup<T, CURVED, MERGE>(fin, PS, p, c, lw, f);
 }
 
 // The links of node c that end on a wall: bounce-back of the node's own
 // f_opp(i), the slip reflection or the curved-wall rule, in place of the pulled
 // value.
-template <typename T, bool CURVED>
+template <typename T, bool CURVED, bool MERGE>
 __device__ __forceinline__ void wall_fixup(const T* __restrict__ fin, size_t PS, const LBKParams& p, const Coord& c,
                                            uint32_t lw, T f[19]) {
     const uint32_t self = (uint32_t)c.idx;
@@ -127,7 +93,7 @@ __device__ __forceinline__ void wall_fixup(const T* __restrict__ fin, size_t PS,
         for (int i = 1; i < 19; ++i) {
             const int j = opp(i);
             if (!(lw & (1u << j))) continue;
-            const T own = ld_pop(&fin[(size_t)j * PS + self]);
+            const T own = ld_pop<MERGE>(&fin[(size_t)j * PS + self]);
             if (CURVED && (cw & (1u << j)))
                 f[i] = curved_link<T, sizeof(T) == 4>(p, c, j, own);
             else if (sw & (1u << j))
@@ -249,7 +215,7 @@ __device__ __forceinline__ void load_prepared(const FSView& fsv, size_t PS, size
 
 // ------------------------------------------------------------------ hydrodynamic run sums
 // Per-slot hydrodynamic sums (LB.cpp:1897-1902) folded into the collision: the
-// workgroup's nodes are 256 consecutive x nodes of one row, so the nodes one
+// nodes of a wavefront are 64 consecutive x nodes of one row, so the nodes one
 // slot owns there form runs. Each particle node stages its penalty increment
 // diffVel and node mass in LDS as the collision computes them (every node first
 // marks its entry empty); at the end the first node of each run adds the run's
@@ -258,8 +224,8 @@ __device__ __forceinline__ void load_prepared(const FSView& fsv, size_t PS, size
 // the slot's list. The per-element combine adds the lists exactly (order-free),
 // so the result does not depend on the order of the appends. Runs end at
 // wavefront boundaries, so only lanes of one wavefront exchange data.
-constexpr int RUN_NODES = 256;  // nodes of one workgroup (one row segment)
-static_assert(BX == RUN_NODES && BY == 1, "run sums need the workgroup on 256 consecutive x nodes of one row");
+constexpr int RUN_NODES = 256;  // nodes of one workgroup
+static_assert(ROW_BLOCK <= RUN_NODES, "one entry per lane of a workgroup");
 
 template <typename DT>
 struct RunLDS {
@@ -287,34 +253,30 @@ struct RunSlot {
     }
 };
 
-// The run sums of a workgroup whose lanes hold NPL consecutive nodes each
-// (node n = NPL * lane + k, x = blockIdx.x * RUN_NODES + n of row (y, z)).
-template <typename DT, int NPL>
+// The run sums of a workgroup, lane n holding node n.
+template <typename DT, bool MERGE>
 __device__ __forceinline__ void hydro_runs(const RunLDS<DT>& L, const HydroSink& hs, const CoupleRec* __restrict__ cp,
                                            const LBKParams& p) {
 #pragma clang fp contract(off)
-    static_assert(RUN_NODES % (64 * NPL) == 0, "workgroup rows of whole wavefronts");
-    constexpr int WAVE_NODES = 64 * NPL;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const int y = (int)blockIdx.y, z = (int)blockIdx.z;
-#pragma unroll
-    for (int k = 0; k < NPL; ++k) {
-        const int n = NPL * (int)threadIdx.x + k;
-        const uint32_t sid = L.sid[n];
-        if (!sid) continue;
-        if (n % WAVE_NODES != 0 && L.sid[n - 1] == sid) continue;  // not the first node of its run
+    const int n = (int)threadIdx.x;
+    const uint32_t sid = L.sid[n];
+    const bool first = sid && (n % 64 == 0 || L.sid[n - 1] != sid);  // of its run
+    if (first) {
+        Coord c;
+        (void)lane_coord<MERGE>(p, c);
         const uint32_t slot = sid - 1;
         const CoupleRec& r = cp[slot];
         const V3 x0(r.x0[0], r.x0[1], r.x0[2]);
         const V3 rv(r.rv[0], r.rv[1], r.rv[2]);
         double acc[7] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-        const int end = (n / WAVE_NODES + 1) * WAVE_NODES;
-        const int xb = (int)blockIdx.x * RUN_NODES;
+        const int end = (n / 64 + 1) * 64;
         for (int m = n; m < end && L.sid[m] == sid; ++m) {
             const V3 d((double)L.d[0][m], (double)L.d[1][m], (double)L.d[2][m]);
-            const V3 radius = V3((double)(xb + m), (double)y, (double)z) - x0 / p.unitLength + rv / p.unitLength;
+            const V3 radius =
+                V3((double)(c.x + (m - n)), (double)c.y, (double)c.z) - x0 / p.unitLength + rv / p.unitLength;
             const V3 mo = radius.cross(d);
             acc[0] += d.x; acc[1] += d.y; acc[2] += d.z;
             acc[3] += mo.x; acc[4] += mo.y; acc[5] += mo.z;
@@ -333,7 +295,7 @@ __device__ __forceinline__ void hydro_runs(const RunLDS<DT>& L, const HydroSink&
     }
 }
 
-template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED = false>
+template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED, bool MERGE>
 __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, double* __restrict__ fout,
                                              const uint32_t* __restrict__ link,
                                              const uint32_t* __restrict__ solid,
@@ -342,16 +304,21 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
                                                      const LBKParams& p, const FSView& fsv) {
 #pragma clang fp contract(off)
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!lane_coord<MERGE>(p, c)) return;
     const size_t N = (size_t)p.X * p.Y * p.Z;
     const uint32_t lw = link[c.idx];
-    if (!(lw & LINK_ACTIVE)) return;
+    const bool act = (lw & LINK_ACTIVE) != 0u;
+    const bool fill = fills_line<double>(act);
+    if (!act && !(fill && fout)) return;
     double f[19];
-    if (FS && (lw & LINK_PRESTREAMED)) load_prepared<double>(fsv, p.PS, c.idx, lw, f);
-    else if (PULL) pull19<double, CURVED>(fin, p.PS, p, c, lw, f);
+    if (!act) {  // any finite collision will do
+#pragma unroll
+        for (int j = 0; j < 19; ++j) f[j] = wgt(j);
+    } else if (FS && (lw & LINK_PRESTREAMED)) load_prepared<double>(fsv, p.PS, c.idx, lw, f);
+    else if (PULL) pull19<double, CURVED, MERGE>(fin, p.PS, p, c, lw, f);
     else {
 #pragma unroll
-        for (int j = 0; j < 19; ++j) f[j] = ld_pop(&fin[(size_t)j * p.PS + c.idx]);
+        for (int j = 0; j < 19; ++j) f[j] = ld_pop<MERGE>(&fin[(size_t)j * p.PS + c.idx]);
     }
     double n;
     V3 u;
@@ -359,7 +326,7 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
     if (p.herr && !isfinite(n)) *p.herr = LB_ERR_NUMERIC;
     // penalty coupling force
     V3 hF(0.0, 0.0, 0.0);
-    const uint32_t sw = solid ? solid[c.idx] : 0u;
+    const uint32_t sw = solid && act ? solid[c.idx] : 0u;
     const uint32_t sid = owner_slot(sw, p.ctag);
     if (sid) {
         const double mass = node_mass<FS, double>(lw, c.idx, fsv, p);
@@ -370,13 +337,13 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
     if (p.ffield) Fb = Fb + V3((double)p.ffield[c.idx], (double)p.ffield[N + c.idx], (double)p.ffield[2 * N + c.idx]);
     const V3 T = Fb + hF;
     u += 0.5 * T / n;  // node.cpp:85-88
-    if (CURVED && p.macNext) {
+    if (CURVED && act && p.macNext) {
         p.macNext[c.idx] = n;
         p.macNext[N + c.idx] = u.x;
         p.macNext[2 * N + c.idx] = u.y;
         p.macNext[3 * N + c.idx] = u.z;
     }
-    if (mac) {
+    if (mac && act) {
         mac[c.idx] = n;
         mac[N + c.idx] = u.x;
         mac[2 * N + c.idx] = u.y;
@@ -386,7 +353,7 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
         mac[6 * N + c.idx] = hF.z;
     }
     if (!fout) return;
-    if (FS) {
+    if (FS && act) {
         ((double*)fsv.rhoCur)[c.idx] = n;
         if (lw & LINK_INTERFACE) {
             fsv.uS[c.idx] = u.x; fsv.uS[N + c.idx] = u.y; fsv.uS[2 * N + c.idx] = u.z;
@@ -404,8 +371,8 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
         double fe[19];
 #pragma unroll
         for (int j = 0; j < 19; ++j) fe[j] = feq(j);
-        nu = shear_visc64(f, fe, n, visc[c.idx], p);
-        visc[c.idx] = nu;
+        nu = shear_visc64(f, fe, n, act ? visc[c.idx] : p.visc0, p);
+        if (act) visc[c.idx] = nu;
     }
     if (COLL == HYB_COLLISION_TRT) {
         const double omP = 1.0 / (0.5 + 3.0 * nu);
@@ -421,7 +388,7 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
             const double cF = cdot_rt(j, T);
             const double sp = wgt(j) * (9.0 * vu * cF - 3.0 * uT);
             const double sm = wgt(j) * (3.0 * cF);
-            st_pop(&fout[(size_t)j * p.PS + c.idx],
+            st_pop<MERGE>(&fout[(size_t)j * p.PS + c.idx],
                    fj - omP * (fp - ep) - omM * (fm - em) + (1.0 - 0.5 * omP) * sp + (1.0 - 0.5 * omM) * sm);
             if (o != j) {
                 // the same expression evaluated for the opposite direction
@@ -431,7 +398,7 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
                 const double cF2 = cdot_rt(o, T);
                 const double sp2 = wgt(o) * (9.0 * vu2 * cF2 - 3.0 * uT);
                 const double sm2 = wgt(o) * (3.0 * cF2);
-                st_pop(&fout[(size_t)o * p.PS + c.idx],
+                st_pop<MERGE>(&fout[(size_t)o * p.PS + c.idx],
                        fo - omP * (fp2 - ep2) - omM * (fm2 - em2) + (1.0 - 0.5 * omP) * sp2 + (1.0 - 0.5 * omM) * sm2);
             }
         }
@@ -447,13 +414,13 @@ __device__ __forceinline__ void fused64_node(const double* __restrict__ fin, dou
             const V3 fp((double)cx(j) * a + ((double)cx(j) - u.x) * 3.0, (double)cy(j) * a + ((double)cy(j) - u.y) * 3.0,
                         (double)cz(j) * a + ((double)cz(j) - u.z) * 3.0);
             fj += 1.0 * omegaf * wgt(j) * fp.dot(T);
-            st_pop(&fout[(size_t)j * p.PS + c.idx], fj);
+            st_pop<MERGE>(&fout[(size_t)j * p.PS + c.idx], fj);
         }
     }
 }
 
-template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED = false>
-__global__ void __launch_bounds__(BX * BY, (VARVISC || CURVED) ? 1 : 5) k_fused64(const double* __restrict__ fin, double* __restrict__ fout,
+template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED, bool MERGE>
+__global__ void __launch_bounds__(ROW_BLOCK, (VARVISC || CURVED) ? 1 : 5) k_fused64(const double* __restrict__ fin, double* __restrict__ fout,
                                                      const uint32_t* __restrict__ link,
                                                      const uint32_t* __restrict__ solid,
                                                      const CoupleRec* __restrict__ cp, HydroSink hs,
@@ -463,8 +430,8 @@ __global__ void __launch_bounds__(BX * BY, (VARVISC || CURVED) ? 1 : 5) k_fused6
     const bool sums = hs.segs != nullptr;
     const RunSlot<double> rs{sums ? &lds : nullptr, (int)threadIdx.x};
     rs.clear();
-    fused64_node<PULL, VARVISC, COLL, FS, CURVED>(fin, fout, link, solid, cp, rs, visc, mac, p, fsv);
-    if (sums) hydro_runs<double, 1>(lds, hs, cp, p);
+    fused64_node<PULL, VARVISC, COLL, FS, CURVED, MERGE>(fin, fout, link, solid, cp, rs, visc, mac, p, fsv);
+    if (sums) hydro_runs<double, MERGE>(lds, hs, cp, p);
 }
 
 // ------------------------------------------------------------------ FP32 deviation path
@@ -478,7 +445,7 @@ __device__ __forceinline__ float cdotf(int j, float ux, float uy, float uz) {
     return r;
 }
 
-// Collision of one node in the FP32 deviation form: moments, penalty force,
+// Collision of one node (act; else a lane that only completes a line, with g of a node at rest) in the FP32 deviation form: moments, penalty force,
 // Guo shift, [Bingham/Smagorinsky], BGK/TRT with Guo forcing. sid: the node's
 // particle slot + 1 (0: none) with that slot's record r. Writes the side
 // outputs (node force, macroscopic fields, viscosity, free-surface state) and,
@@ -487,7 +454,7 @@ __device__ __forceinline__ float cdotf(int j, float ux, float uy, float uz) {
 // caller reports it), so that no global store sits between the loads of the
 // nodes of one lane.
 template <bool VARVISC, int COLL, bool FS, bool CURVED = false>
-__device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uint32_t lw, size_t N, uint32_t sid,
+__device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uint32_t lw, bool act, size_t N, uint32_t sid,
                                           const CoupleRecF& r, const RunSlot<float>& rs, double* __restrict__ visc,
                                           double* __restrict__ mac, const LBKParams& p, const FSView& fsv, bool doOut,
                                           float out[19], bool& bad) {
@@ -531,13 +498,13 @@ __device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uin
     ux += 0.5f * Tx * irho;
     uy += 0.5f * Ty * irho;
     uz += 0.5f * Tz * irho;
-    if (CURVED && p.macNext) {
+    if (CURVED && act && p.macNext) {
         p.macNext[c.idx] = (double)rho;
         p.macNext[N + c.idx] = ux;
         p.macNext[2 * N + c.idx] = uy;
         p.macNext[3 * N + c.idx] = uz;
     }
-    if (mac) {
+    if (mac && act) {
         mac[c.idx] = (double)rho;
         mac[N + c.idx] = ux;
         mac[2 * N + c.idx] = uy;
@@ -547,7 +514,7 @@ __device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uin
         mac[6 * N + c.idx] = hz;
     }
     if (!doOut) return false;
-    if (FS) {
+    if (FS && act) {
         ((float*)fsv.rhoCur)[c.idx] = rho;
         if (lw & LINK_INTERFACE) {
             fsv.uS[c.idx] = ux; fsv.uS[N + c.idx] = uy; fsv.uS[2 * N + c.idx] = uz;
@@ -575,7 +542,7 @@ __device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uin
             if (cz(j) * cx(j) > 0) s[5] += d;
             if (cz(j) * cx(j) < 0) s[5] -= d;
         }
-        const double viscOld = visc[c.idx];
+        const double viscOld = act ? visc[c.idx] : p.visc0;
         const float tau = 0.5f + 3.0f * (float)viscOld;
         const float k = 1.5f / (tau * rho);
         const float g00 = s[0] * k, g11 = s[1] * k, g22 = s[2] * k, g01 = s[3] * k, g12 = s[4] * k, g20 = s[5] * k;
@@ -590,7 +557,7 @@ __device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uin
         const float maxV = (float)((1.8 - 0.5) / 3.0), minV = (float)((0.501 - 0.5) / 3.0);
         const float lo = (a < maxV) ? a : maxV;
         nu = (minV < lo) ? lo : minV;
-        visc[c.idx] = (double)nu;
+        if (act) visc[c.idx] = (double)nu;
     }
     const float omP = 1.0f / (0.5f + 3.0f * nu);
     const float uT = ux * Tx + uy * Ty + uz * Tz;
@@ -624,39 +591,47 @@ __device__ __forceinline__ bool collide32(const float g[19], const Coord& c, uin
 }
 
 
-template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED = false>
+template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED, bool MERGE>
 __device__ __forceinline__ void fused32_node(const float* __restrict__ fin, float* __restrict__ fout,
                                              const uint32_t* __restrict__ link, const uint32_t* __restrict__ solid,
                                              const CoupleRecF* __restrict__ cp, const RunSlot<float>& rs,
                                              double* __restrict__ visc, double* __restrict__ mac, const LBKParams& p,
                                              const FSView& fsv) {
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!lane_coord<MERGE>(p, c)) return;
     const size_t N = (size_t)p.X * p.Y * p.Z;
     const uint32_t lw = link[c.idx];
-    if (!(lw & LINK_ACTIVE)) return;
+    const bool act = (lw & LINK_ACTIVE) != 0u;
+    const bool fill = fills_line<float>(act);
+    if (!act && !(fill && fout)) return;
     float g[19];
-    if (FS && (lw & LINK_PRESTREAMED)) load_prepared<float>(fsv, p.PS, c.idx, lw, g);
-    else if (PULL) pull19<float, CURVED>(fin, p.PS, p, c, lw, g);
-    else {
-#pragma unroll
-        for (int j = 0; j < 19; ++j) g[j] = ld_pop(&fin[(size_t)j * p.PS + c.idx]);
-    }
-    const uint32_t sid = owner_slot(solid ? solid[c.idx] : 0u, p.ctag);
+    uint32_t sid = 0u;
     CoupleRecF r{};
-    if (sid) r = cp[sid - 1];
+    if (act) {
+        if (FS && (lw & LINK_PRESTREAMED)) load_prepared<float>(fsv, p.PS, c.idx, lw, g);
+        else if (PULL) pull19<float, CURVED, MERGE>(fin, p.PS, p, c, lw, g);
+        else {
+#pragma unroll
+            for (int j = 0; j < 19; ++j) g[j] = ld_pop<MERGE>(&fin[(size_t)j * p.PS + c.idx]);
+        }
+        sid = owner_slot(solid ? solid[c.idx] : 0u, p.ctag);
+        if (sid) r = cp[sid - 1];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 19; ++j) g[j] = 0.0f;
+    }
     float out[19];
     bool bad;
-    const bool wrote = collide32<VARVISC, COLL, FS, CURVED>(g, c, lw, N, sid, r, rs, visc, mac, p, fsv,
+    const bool wrote = collide32<VARVISC, COLL, FS, CURVED>(g, c, lw, act, N, sid, r, rs, visc, mac, p, fsv,
                                                            fout != nullptr, out, bad);
     if (bad && p.herr) *p.herr = LB_ERR_NUMERIC;
     if (!wrote) return;
 #pragma unroll
-    for (int j = 0; j < 19; ++j) st_pop(&fout[(size_t)j * p.PS + c.idx], out[j]);
+    for (int j = 0; j < 19; ++j) st_pop<MERGE>(&fout[(size_t)j * p.PS + c.idx], out[j]);
 }
 
-template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED = false>
-__global__ void __launch_bounds__(BX * BY, (VARVISC || CURVED) ? 1 : 8) k_fused32(const float* __restrict__ fin, float* __restrict__ fout,
+template <bool PULL, bool VARVISC, int COLL, bool FS, bool CURVED, bool MERGE>
+__global__ void __launch_bounds__(ROW_BLOCK, (VARVISC || CURVED) ? 1 : 8) k_fused32(const float* __restrict__ fin, float* __restrict__ fout,
                                                      const uint32_t* __restrict__ link,
                                                      const uint32_t* __restrict__ solid,
                                                      const CoupleRecF* __restrict__ cp, const CoupleRec* __restrict__ cp64,
@@ -666,22 +641,22 @@ __global__ void __launch_bounds__(BX * BY, (VARVISC || CURVED) ? 1 : 8) k_fused3
     const bool sums = hs.segs != nullptr;
     const RunSlot<float> rs{sums ? &lds : nullptr, (int)threadIdx.x};
     rs.clear();
-    fused32_node<PULL, VARVISC, COLL, FS, CURVED>(fin, fout, link, solid, cp, rs, visc, mac, p, fsv);
-    if (sums) hydro_runs<float, 1>(lds, hs, cp64, p);
+    fused32_node<PULL, VARVISC, COLL, FS, CURVED, MERGE>(fin, fout, link, solid, cp, rs, visc, mac, p, fsv);
+    if (sums) hydro_runs<float, MERGE>(lds, hs, cp64, p);
 }
 
 // Standalone pull streaming: turns the post-collision state into the
 // reference's step-end (post-stream) populations, for host views only.
 template <typename T, bool CURVED = false>
-__global__ void __launch_bounds__(BX * BY) k_stream(const T* __restrict__ fin, T* __restrict__ fout,
+__global__ void __launch_bounds__(ROW_BLOCK) k_stream(const T* __restrict__ fin, T* __restrict__ fout,
                                                     const uint32_t* __restrict__ link, LBKParams p) {
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     const size_t N = (size_t)p.X * p.Y * p.Z;
     const uint32_t lw = link[c.idx];
     if (!(lw & LINK_ACTIVE)) return;
     T f[19];
-    pull19<T, CURVED>(fin, p.PS, p, c, lw, f);
+    pull19<T, CURVED, false>(fin, p.PS, p, c, lw, f);
 #pragma unroll
     for (int j = 0; j < 19; ++j) fout[(size_t)j * p.PS + c.idx] = f[j];
 }
@@ -695,7 +670,7 @@ __global__ void k_init_types(uint8_t* __restrict__ type, LBKParams p, int b0, in
                              CylSet cs, int problem, double lx0, double lx1, double ly0, double ly1, double lz0,
                              double lz1, double avalanchePosit) {
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     uint8_t t = T_FLUID;
     auto isWall = [](uint8_t tt) { return tt == 5 || tt == 6 || tt == 7 || tt == 8 || tt == 9; };
     if (c.x == 0 && !isWall(t)) t = (uint8_t)b0;
@@ -751,7 +726,7 @@ __global__ void k_init_types(uint8_t* __restrict__ type, LBKParams p, int b0, in
 // because neither loop changes the property it tests on its neighbours.
 __global__ void k_tag_interface(const uint8_t* __restrict__ tin, uint8_t* __restrict__ tout, LBKParams p) {
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     uint8_t t = tin[c.idx];
     if (t == T_FLUID && interior(p, c)) {
         for (int j = 1; j < 19; ++j)
@@ -763,7 +738,7 @@ __global__ void k_tag_interface(const uint8_t* __restrict__ tin, uint8_t* __rest
 // Isolated interface nodes become gas (LB.cpp:799-814).
 __global__ void k_remove_isolated(const uint8_t* __restrict__ tin, uint8_t* __restrict__ tout, LBKParams p) {
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     uint8_t t = tin[c.idx];
     if (t == T_INTERFACE && interior(p, c)) {
         bool close = false;
@@ -777,7 +752,7 @@ __global__ void k_remove_isolated(const uint8_t* __restrict__ tin, uint8_t* __re
 __global__ void k_init_links(const uint8_t* __restrict__ type, uint32_t* __restrict__ link, uint32_t* __restrict__ slipw,
                              uint32_t* __restrict__ curvw, LBKParams p) {
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     const uint8_t t = type[c.idx];
     uint32_t lw = 0, sw = 0, cw = 0;
     if ((t == T_FLUID || t == T_INTERFACE) && interior(p, c)) {
@@ -802,7 +777,7 @@ __global__ void k_init_links(const uint8_t* __restrict__ type, uint32_t* __restr
 __global__ void k_max_active(const uint32_t* __restrict__ link, int* __restrict__ mx, LBKParams p) {
     Coord c;
     int v[3] = {-1, -1, -1};
-    if (node_coord(p, c) && (link[c.idx] & LINK_ACTIVE)) { v[0] = c.x; v[1] = c.y; v[2] = c.z; }
+    if (row_coord(p, c) && (link[c.idx] & LINK_ACTIVE)) { v[0] = c.x; v[1] = c.y; v[2] = c.z; }
     for (int k = 0; k < 3; ++k) {
         int m = v[k];
         for (int off = 32; off > 0; off >>= 1) {
@@ -822,7 +797,7 @@ __global__ void k_init_pops(T* __restrict__ f, const uint32_t* __restrict__ link
                             double* __restrict__ uS) {
 #pragma clang fp contract(off)
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     const size_t N = (size_t)p.X * p.Y * p.Z;
     const uint32_t lw = link[c.idx];
     if (!(lw & LINK_ACTIVE)) return;
@@ -858,7 +833,7 @@ __global__ void k_init_pops(T* __restrict__ f, const uint32_t* __restrict__ link
 __global__ void k_count_active(const uint32_t* __restrict__ link, unsigned long long* __restrict__ cnt, LBKParams p) {
     Coord c;
     bool a = false;
-    if (node_coord(p, c)) a = (link[c.idx] & LINK_ACTIVE) != 0;
+    if (row_coord(p, c)) a = (link[c.idx] & LINK_ACTIVE) != 0;
     const unsigned long long b = __ballot(a);
     // one counter per z-plane; the host adds the planes
     if ((threadIdx.x & 63) == 0 && b) atomicAdd(&cnt[blockIdx.z], (unsigned long long)__popcll(b));
@@ -870,7 +845,7 @@ __global__ void k_count_mass(const uint32_t* __restrict__ link, const uint32_t* 
                              unsigned long long* __restrict__ cnt, LBKParams p) {
     Coord c;
     bool fl = false, in = false;
-    if (node_coord(p, c)) {
+    if (row_coord(p, c)) {
         const uint32_t lw = link[c.idx];
         const bool owned = solid && owner_slot(solid[c.idx], p.ctag) != 0u;
         fl = (lw & LINK_ACTIVE) && !(lw & LINK_INTERFACE) && !owned;
@@ -1040,12 +1015,12 @@ __global__ void __launch_bounds__(256) k_classify_set(const int* __restrict__ ns
 // fs is the post-collision state of the last step. Exact fixed-point sums:
 // acc[(wall * 3 + k) * 4 ...].
 template <typename T, bool SHIFT>
-__global__ void __launch_bounds__(BX * BY) k_wall_fhydro(const T* __restrict__ f, const uint8_t* __restrict__ type,
+__global__ void __launch_bounds__(ROW_BLOCK) k_wall_fhydro(const T* __restrict__ f, const uint8_t* __restrict__ type,
                                                           WallSet ws, unsigned long long* __restrict__ acc,
                                                           LBKParams p) {
 #pragma clang fp contract(off)
     Coord c;
-    if (!node_coord(p, c)) return;
+    if (!row_coord(p, c)) return;
     const uint8_t t = type[c.idx];
     if (t != T_FLUID && t != T_INTERFACE) return;
     for (int j = 1; j < 19; ++j) {
@@ -1107,40 +1082,40 @@ __global__ void k_fill_u32(uint32_t* __restrict__ a, uint32_t v, size_t n) {
     if (i < n) a[i] = v;
 }
 
-dim3 lattice_grid(const LBKParams& p) { return dim3((p.X + BX - 1) / BX, (p.Y + BY - 1) / BY, p.Z); }
-
 }  // namespace
 
 // ------------------------------------------------------------------ launchers
-#define HYB_FUSED_LAUNCH(PULL, VV, CO, CUR)                                                                        \
+#define HYB_FUSED_LAUNCH(PULL, VV, CO, CUR, MERGE)                                                                   \
     if (pull == PULL && varVisc == VV && collision == CO) {                                                        \
         if (prec == Prec::F64) {                                                                                   \
             if (fs)                                                                                                \
-                k_fused64<PULL, VV, CO, true, CUR><<<g, b, 0, s>>>((const double*)fin, (double*)fout, link, solid, \
-                                                                   cp, sink, visc, mac, p, *fs);                   \
+                k_fused64<PULL, VV, CO, true, CUR, MERGE><<<g, b, 0, s>>>((const double*)fin, (double*)fout, link,  \
+                                                                         solid, cp, sink, visc, mac, p, *fs);      \
             else                                                                                                   \
-                k_fused64<PULL, VV, CO, false, CUR><<<g, b, 0, s>>>((const double*)fin, (double*)fout, link,       \
-                                                                    solid, cp, sink, visc, mac, p, none);          \
+                k_fused64<PULL, VV, CO, false, CUR, MERGE><<<g, b, 0, s>>>((const double*)fin, (double*)fout, link, \
+                                                                          solid, cp, sink, visc, mac, p, none);    \
         } else {                                                                                                   \
             if (fs)                                                                                                \
-                k_fused32<PULL, VV, CO, true, CUR><<<g, b, 0, s>>>((const float*)fin, (float*)fout, link, solid,   \
-                                                                   cpf, cp, sink, visc, mac, p, *fs);              \
+                k_fused32<PULL, VV, CO, true, CUR, MERGE><<<g, b, 0, s>>>(                                          \
+                    (const float*)fin, (float*)fout, link, solid, cpf, cp, sink, visc, mac, p, *fs);               \
             else                                                                                                   \
-                k_fused32<PULL, VV, CO, false, CUR><<<g, b, 0, s>>>((const float*)fin, (float*)fout, link, solid,  \
-                                                                    cpf, cp, sink, visc, mac, p, none);            \
+                k_fused32<PULL, VV, CO, false, CUR, MERGE><<<g, b, 0, s>>>(                                         \
+                    (const float*)fin, (float*)fout, link, solid, cpf, cp, sink, visc, mac, p, none);              \
         }                                                                                                          \
         return;                                                                                                    \
     }
 // Cylinders (p.curvw set, CUR = true): the curved-wall pull and the capture of
 // every active node's density and velocity for the next step's curved links.
-#define HYB_FUSED_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, false)
-#define HYB_CURVED_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, true)
+#define HYB_FUSED_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, false, false)
+#define HYB_MERGE_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, false, true)
+#define HYB_CURVED_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, true, false)
 
 void launch_lb_fused(Prec prec, bool pull, bool varVisc, int collision, const void* fin, void* fout,
                      const uint32_t* link, const uint32_t* solid, const CoupleRec* cp, const CoupleRecF* cpf,
                      const HydroSink* hs, double* visc, double* mac, const FSView* fs, const LBKParams& p,
                      hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const bool merge = !p.curvw && merge_map(p, prec);
+    const dim3 g = merge ? merge_grid(p) : row_grid(p), b = row_block(p);
     const FSView none{};
     const HydroSink sink = (hs && solid) ? *hs : HydroSink{nullptr, nullptr, 0u};
     if (p.curvw) {
@@ -1152,6 +1127,16 @@ void launch_lb_fused(Prec prec, bool pull, bool varVisc, int collision, const vo
         HYB_CURVED_CASE(false, false, HYB_COLLISION_TRT)
         HYB_CURVED_CASE(false, true, HYB_COLLISION_BGK)
         HYB_CURVED_CASE(false, true, HYB_COLLISION_TRT)
+    }
+    if (merge) {
+        HYB_MERGE_CASE(true, false, HYB_COLLISION_BGK)
+        HYB_MERGE_CASE(true, false, HYB_COLLISION_TRT)
+        HYB_MERGE_CASE(true, true, HYB_COLLISION_BGK)
+        HYB_MERGE_CASE(true, true, HYB_COLLISION_TRT)
+        HYB_MERGE_CASE(false, false, HYB_COLLISION_BGK)
+        HYB_MERGE_CASE(false, false, HYB_COLLISION_TRT)
+        HYB_MERGE_CASE(false, true, HYB_COLLISION_BGK)
+        HYB_MERGE_CASE(false, true, HYB_COLLISION_TRT)
     }
     HYB_FUSED_CASE(true, false, HYB_COLLISION_BGK)
     HYB_FUSED_CASE(true, false, HYB_COLLISION_TRT)
@@ -1165,7 +1150,7 @@ void launch_lb_fused(Prec prec, bool pull, bool varVisc, int collision, const vo
 
 void launch_wall_fhydro(Prec prec, const void* f, const uint8_t* type, const WallSet& ws, unsigned long long* acc,
                         const LBKParams& p, hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     if (prec == Prec::F64) k_wall_fhydro<double, false><<<g, b, 0, s>>>((const double*)f, type, ws, acc, p);
     else k_wall_fhydro<float, true><<<g, b, 0, s>>>((const float*)f, type, ws, acc, p);
 }
@@ -1226,7 +1211,7 @@ void launch_status(const double* mac, const double* visc, const uint32_t* link, 
 }
 
 void launch_lb_stream(Prec prec, const void* fin, void* fout, const uint32_t* link, const LBKParams& p, hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     if (p.curvw) {
         if (prec == Prec::F64) k_stream<double, true><<<g, b, 0, s>>>((const double*)fin, (double*)fout, link, p);
         else k_stream<float, true><<<g, b, 0, s>>>((const float*)fin, (float*)fout, link, p);
@@ -1239,31 +1224,31 @@ void launch_lb_stream(Prec prec, const void* fin, void* fout, const uint32_t* li
 void launch_lb_init_types(uint8_t* type, const int* bnd, int nwalls, const WallDev* walls, int nobj,
                           const ObjDev* objs, const CylSet& cs, int problem, const double* lbx, const LBKParams& p,
                           hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     k_init_types<<<g, b, 0, s>>>(type, p, bnd[0], bnd[1], bnd[2], bnd[3], bnd[4], bnd[5], nwalls, walls, nobj, objs,
                                  cs, problem, lbx[0], lbx[1], lbx[2], lbx[3], lbx[4], lbx[5], lbx[6]);
 }
 
 void launch_lb_init_interface(uint8_t* type, uint8_t* tmp, const LBKParams& p, hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     k_tag_interface<<<g, b, 0, s>>>(type, tmp, p);
     k_remove_isolated<<<g, b, 0, s>>>(tmp, type, p);
 }
 
 void launch_lb_init_links(const uint8_t* type, uint32_t* link, uint32_t* slipw, uint32_t* curvw, const LBKParams& p,
                           hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     k_init_links<<<g, b, 0, s>>>(type, link, slipw, curvw, p);
 }
 
 void launch_lb_max_active(const uint32_t* link, int* mx, const LBKParams& p, hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     k_max_active<<<g, b, 0, s>>>(link, mx, p);
 }
 
 void launch_lb_init_pops(Prec prec, void* f, const uint32_t* link, const int* mx, double* visc, const double* u0,
                          const double* Finit, void* rho, double* mass, double* uS, const LBKParams& p, hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     if (prec == Prec::F64)
         k_init_pops<double, false><<<g, b, 0, s>>>((double*)f, link, mx, visc, p, u0[0], u0[1], u0[2], Finit[0],
                                                    Finit[1], Finit[2], (double*)rho, mass, uS);
@@ -1288,12 +1273,12 @@ void launch_fill_u32(uint32_t* a, uint32_t v, size_t n, hipStream_t s) {
 
 void launch_count_mass(const uint32_t* link, const uint32_t* solid, unsigned long long* count, const LBKParams& p,
                        hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     k_count_mass<<<g, b, 0, s>>>(link, solid, count, p);
 }
 
 void launch_count_active(const uint32_t* link, unsigned long long* count, const LBKParams& p, hipStream_t s) {
-    const dim3 g = lattice_grid(p), b(BX, BY, 1);
+    const dim3 g = row_grid(p), b = row_block(p);
     k_count_active<<<g, b, 0, s>>>(link, count, p);
 }
 

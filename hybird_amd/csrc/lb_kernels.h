@@ -49,6 +49,7 @@ struct LBKParams {
     // the handle's error word (mapped pinned host memory; nullptr: none): a
     // collision that finds a non-finite density stores LB_ERR_NUMERIC there
     int* herr;
+    uint64_t invRows, invChunks;  // inverse_of the workgroups of a z plane, of a row (merge_coord)
 };
 
 constexpr int LB_ERR_NUMERIC = 6;
