@@ -39,7 +39,20 @@ namespace {
 
 constexpr int FS_BLOCK = 256;
 constexpr int FS_GRID = 1024;
+// k_fs_mass: one wavefront per workgroup, so that a short list reaches more CUs (3,600 nodes 27 -> 12 us, 31,000
+// nodes 43 -> 33, 262,144 nodes 31 -> 33)
+constexpr int MASS_BLOCK = 64, MASS_GRID = FS_GRID * FS_BLOCK / MASS_BLOCK;
+// Passes between two orderings of the interface list (k_fs_build_list). us a cycle over 200 cycles, every pass / 8 / 32 /
+// never: 262,144 interface nodes of 512 x 512 x 256 1580 to 1593 / 1565 to 1583 / 1566 to 1591 / 1569 to 1656 and
+// rising, 31,000 of 384 x 128 x 192 336 / 319 / 316 / 316, 3,600 of 101 x 47 x 66 149 / 146 / 146 / 143.
+constexpr uint32_t SORT_STEPS = 16;
 enum : uint8_t { FS_STAY = 0, FS_FILLED = 1, FS_EMPTIED = 2 };
+
+// Adds the lanes' sums to the accumulator: most wavefronts have none, the others one atomic per limb instead of one
+// per node (atomics on one address take about 10 ns each, over all XCDs).
+__device__ __forceinline__ void flush_acc(unsigned long long* acc, long long s[4]) {
+    if (__any((s[0] | s[1] | s[2] | s[3]) != 0)) exact_flush(acc, s);
+}
 
 #define FS_FOR(i, n) \
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += gridDim.x * blockDim.x)
@@ -52,8 +65,76 @@ __device__ __forceinline__ double to_d(T v) {
 // ---- 1. streaming of the interface nodes + updateMass (LB.cpp:1492-1590)
 // SHIFT: populations are stored as f - w (rho0 = 1); f_opp - fs_j is the same in
 // both forms because w_opp(j) = w_j.
+//
+// What link j of a node brings: the population v streamed in against j and the share a of the mass exchange. tl, vn
+// and mL: the neighbour's type, its population opp(j) (only used with pull) and its mass.
+struct MassNode {
+    size_t idx;
+    Coord c;
+    V3 u;
+    double usq, mi;
+};
+// Links to anything but slip walls and cylinders, after a collision.
+__device__ __forceinline__ bool plain_link(uint8_t tl) { return !is_slip_wall(tl) && tl != T_CURVED; }
 template <typename T, bool SHIFT>
-__global__ void __launch_bounds__(FS_BLOCK)
+__device__ __forceinline__ T link_in(int j, uint8_t tl, T fsj, T vn, double mL, const MassNode& nd, double rho0, double& a) {
+#pragma clang fp contract(off)
+    a = 0.0;
+    if (tl == T_FLUID || tl == T_INTERFACE) {
+        a = (tl == T_INTERFACE) ? 0.5 * (mL + nd.mi) : 1.0;
+        return vn;  // fpost[opp][L], LB.cpp:1234
+    }
+    if (tl == T_GAS) {
+        // LB.cpp:1237-1246 with the shifted velocity of the last collision
+        const double vu = nd.u.dot(V3((double)cx(j), (double)cy(j), (double)cz(j)));
+        const double g = wgt(j) * rho0 * (2.0 + 9.0 * (vu * vu) - 3.0 * nd.usq);
+        return SHIFT ? (T)(-to_d(fsj) + (g - 2.0 * wgt(j))) : (T)(-to_d(fsj) + g);
+    }
+    if (tl == T_WALL_MOVING) a = 1.0 * nd.mi;  // zero velocity, so half-way bounce-back as at a static wall
+    return fsj;
+}
+// Any link, in the pull form or before the first collision (f = fs).
+template <typename T, bool SHIFT>
+__device__ __forceinline__ T any_link(int j, bool pull, uint8_t tl, T fsj, const T* __restrict__ fpost,
+                                      const uint8_t* __restrict__ type, const double* __restrict__ mass, const MassNode& nd,
+                                      const LBKParams& p, double& a) {
+#pragma clang fp contract(off)
+    const double mi = nd.mi;
+    const auto active = [&](size_t n) { const uint8_t t = type[n]; return t == T_FLUID || t == T_INTERFACE; };
+    // moving walls have zero velocity. Mass exchange: a = m for a moving wall, the slip rule for a moving slip wall
+    // (LB.cpp:1531-1575), else 0.
+    const auto slip_share = [&]() {
+        bool half = false;
+        if (j > 6) {
+            const bool a1 = active(nb_index(p, nd.c, slip1check(j))), a2 = active(nb_index(p, nd.c, slip2check(j)));
+            half = (a1 && !a2) || (!a1 && a2);
+        }
+        return half ? 0.0 + 1.0 * p.slipS2 * mi : 0.0 + 1.0 * mi;
+    };
+    const size_t L = nb_index(p, nd.c, j);
+    if (pull && plain_link(tl))
+        return link_in<T, SHIFT>(j, tl, fsj, fpost[(size_t)opp(j) * p.PS + L], mass[L], nd, p.initDensity, a);
+    a = 0.0;
+    if (tl == T_WALL_MOVING) a = 1.0 * mi;
+    else if (tl == T_SLIP_MOVING) a = slip_share();
+    else if (tl == T_CURVED) a = 1.0 * mi;  // LB.cpp:1539-1545
+    if (!pull) {
+        if (tl == T_INTERFACE) a = 0.5 * (mass[L] + mi);
+        else if (tl == T_FLUID) a = 1.0;
+        return fpost[(size_t)opp(j) * p.PS + nd.idx];
+    }
+    // plane wall: bounce-back, slip reflection (LB.cpp:1321-1456); cylinder: Mei-Luo-Shyy (LB.cpp:1278-1319)
+    if (tl == T_CURVED) return curved_link<T, SHIFT>(p, nd.c, j, fsj);
+    if (is_slip_wall(tl)) return wall_link<T>(fpost, p.PS, p, nd.c, true, j, fsj, active);
+    return fsj;
+}
+
+// Bound by memory latency and by the lines it touches: about 400 bytes a node where neighbouring lanes hold
+// neighbouring nodes (FP32: 262,144 nodes of one z plane 147 us with the list as the atomics left it and one
+// wavefront per SIMD, 33 now). PLAIN: after a collision, in a lattice without slip walls and cylinders; otherwise links are
+// taken one at a time (unrolled as well, those rules left one wavefront per SIMD).
+template <typename T, bool SHIFT, bool PLAIN>
+__global__ void __launch_bounds__(MASS_BLOCK, PLAIN ? (sizeof(T) == 4 ? 4 : 3) : 1)
     k_fs_mass(const T* __restrict__ fpost, T* __restrict__ fout, const uint8_t* __restrict__ type,
               const double* __restrict__ mass, const T* __restrict__ rho, const double* __restrict__ uS,
               const uint32_t* __restrict__ list, FSCounters* __restrict__ ctr, int cur, double* __restrict__ mnew,
@@ -68,98 +149,67 @@ __global__ void __launch_bounds__(FS_BLOCK)
         for (int i = 0; i < 4; ++i) ctr->acc[i] = 0ull;
         for (int i = 0; i < 4; ++i) ctr->tot[i] = 0ull;
     }
-    const double rho0 = p.initDensity;
+    const uint32_t sX = (uint32_t)p.X, sXY = (uint32_t)p.X * (uint32_t)p.Y;
     FS_FOR(pos, nI) {
-        const size_t idx = list[pos];
-        const Coord c = coord_of(p, idx);
-        T fs[19], fi[19];
-#pragma unroll
-        for (int j = 0; j < 19; ++j) fs[j] = fpost[(size_t)j * p.PS + idx];
-        const double mi = mass[idx];
-        const V3 u(uS[idx], uS[N + idx], uS[2 * N + idx]);
+        MassNode nd;
+        nd.idx = list[pos];
+        nd.c = coord_of(p, nd.idx);
+        const size_t idx = nd.idx;
+        const Nb3 nx = nb3(nd.c.x, p.X, p.per[0]), ny = nb3(nd.c.y, p.Y, p.per[1]), nz = nb3(nd.c.z, p.Z, p.per[2]);
+        const auto nb = [&](int j) {
+            return (uint32_t)pick(nx, cx(j)) + sX * (uint32_t)pick(ny, cy(j)) + sXY * (uint32_t)pick(nz, cz(j));
+        };
         if (p.actPrev) {  // type class before this pass of the nodes it may change
             uint32_t* ap = const_cast<uint32_t*>(p.actPrev);
             ap[idx] = (p.actTag << 2) | 2u;
             for (int j = 1; j < 19; ++j) {
-                const size_t L = nb_index(p, c, j);
+                const size_t L = nb_index(p, nd.c, j);
                 if (type[L] == T_GAS) ap[L] = p.actTag << 2;
             }
         }
-        const double usq = u.norm2();
-        // every neighbour's type and mass, and in the pull form its opposite population, loaded
-        // together before any is used (a neighbour index is always a node of the lattice, so the loads a
-        // neighbour's type makes unnecessary stay in bounds): one round trip instead of one per link
-        uint8_t tn[19];
-        T vn[19];
-        double mL[19];
-#pragma unroll
-        for (int j = 1; j < 19; ++j) {
-            const size_t L = nb_index(p, c, j);
-            tn[j] = type[L];
-            vn[j] = pull ? fpost[(size_t)opp(j) * p.PS + L] : (T)0;
-            mL[j] = mass[L];
-        }
-        fi[0] = fs[0];
+        nd.mi = mass[idx];
+        nd.u = V3(uS[idx], uS[N + idx], uS[2 * N + idx]);
+        nd.usq = nd.u.norm2();
         double dm = 0.0;
+        if constexpr (PLAIN) {
+            // every neighbour's type and mass and its opposite population, loaded together before any is used (a
+            // neighbour index is always a node of the lattice, so the loads a neighbour's type makes unnecessary
+            // stay in bounds): one round trip instead of one per link
+            T fs[19], vn[19];
+            uint8_t tn[19];
+            double mL[19];
 #pragma unroll
-        for (int j = 1; j < 19; ++j) {
-            const int o = opp(j);
-            const uint8_t tl = tn[j];
-            double a = 0.0;
-            T v;
-            if (!pull) {
-                v = fs[o];  // before the first collision f = fs
-                if (tl == T_INTERFACE) a = 0.5 * (mL[j] + mi);
-                else if (tl == T_FLUID) a = 1.0;
-                else if (tl == T_WALL_MOVING || tl == T_CURVED) a = 1.0 * mi;
-                else if (tl == T_SLIP_MOVING) {
-                    const auto active = [&](size_t n) { const uint8_t t = type[n]; return t == T_FLUID || t == T_INTERFACE; };
-                    bool half = false;
-                    if (j > 6) {
-                        const bool a1 = active(nb_index(p, c, slip1check(j))), a2 = active(nb_index(p, c, slip2check(j)));
-                        half = (a1 && !a2) || (!a1 && a2);
-                    }
-                    a = half ? 0.0 + 1.0 * p.slipS2 * mi : 0.0 + 1.0 * mi;
-                }
-            } else if (tl == T_FLUID || tl == T_INTERFACE) {
-                v = vn[j];  // fpost[opp][L], LB.cpp:1234
-                a = (tl == T_INTERFACE) ? 0.5 * (mL[j] + mi) : 1.0;
-            } else if (tl == T_GAS) {
-                // LB.cpp:1237-1246 with the shifted velocity of the last collision
-                const double vu = u.dot(V3((double)cx(j), (double)cy(j), (double)cz(j)));
-                const double g = wgt(j) * rho0 * (2.0 + 9.0 * (vu * vu) - 3.0 * usq);
-                if (SHIFT) v = (T)(-to_d(fs[j]) + (g - 2.0 * wgt(j)));
-                else v = (T)(-to_d(fs[j]) + g);
-            } else {
-                // plane wall: bounce-back, slip reflection (LB.cpp:1321-1456); moving
-                // walls have zero velocity. Mass exchange: a = m for a moving wall,
-                // the slip rule for a moving slip wall (LB.cpp:1531-1575), else 0.
-                v = fs[j];
-                const auto active = [&](size_t n) { const uint8_t t = type[n]; return t == T_FLUID || t == T_INTERFACE; };
-                if (is_slip_wall(tl)) v = wall_link<T>(fpost, p.PS, p, c, true, j, fs[j], active);
-                if (tl == T_CURVED) {  // Mei-Luo-Shyy (LB.cpp:1278-1319), a = m (LB.cpp:1539-1545)
-                    v = curved_link<T, SHIFT>(p, c, j, fs[j]);
-                    a = 1.0 * mi;
-                } else if (tl == T_WALL_MOVING) {
-                    a = 1.0 * mi;
-                } else if (tl == T_SLIP_MOVING) {
-                    bool half = false;
-                    if (j > 6) {
-                        const bool a1 = active(nb_index(p, c, slip1check(j))), a2 = active(nb_index(p, c, slip2check(j)));
-                        half = (a1 && !a2) || (!a1 && a2);
-                    }
-                    a = half ? 0.0 + 1.0 * p.slipS2 * mi : 0.0 + 1.0 * mi;
-                }
+            for (int j = 0; j < 19; ++j) fs[j] = fpost[(size_t)j * p.PS + idx];
+#pragma unroll
+            for (int j = 1; j < 19; ++j) {
+                const uint32_t L = nb(j);
+                tn[j] = type[L];
+                vn[j] = fpost[(size_t)opp(j) * p.PS + L];
+                mL[j] = mass[L];
             }
-            fi[o] = v;
-            dm += 1.0 * a * (to_d(v) - to_d(fs[j]));
+            fout[idx] = fs[0];
+#pragma unroll
+            for (int j = 1; j < 19; ++j) {
+                double a;
+                const T v = link_in<T, SHIFT>(j, tn[j], fs[j], vn[j], mL[j], nd, p.initDensity, a);
+                fout[(size_t)opp(j) * p.PS + idx] = v;
+                dm += 1.0 * a * (to_d(v) - to_d(fs[j]));
+            }
+        } else {
+            fout[idx] = fpost[idx];
+#pragma unroll 1
+            for (int j = 1; j < 19; ++j) {
+                double a;
+                const T fsj = fpost[(size_t)j * p.PS + idx];
+                const T v = any_link<T, SHIFT>(j, pull != 0, type[nb_index(p, nd.c, j)], fsj, fpost, type, mass, nd, p, a);
+                fout[(size_t)opp(j) * p.PS + idx] = v;
+                dm += 1.0 * a * (to_d(v) - to_d(fsj));
+            }
         }
-        const double mn = mi + dm;
+        const double mn = nd.mi + dm;
         const double n = to_d(rho[idx]);
         state[pos] = mn > n ? FS_FILLED : (mn < 0.0 ? FS_EMPTIED : FS_STAY);
         mnew[pos] = mn;
-#pragma unroll
-        for (int j = 0; j < 19; ++j) fout[(size_t)j * p.PS + idx] = fi[j];
     }
 }
 
@@ -199,34 +249,46 @@ __global__ void __launch_bounds__(FS_BLOCK)
 #pragma clang fp contract(off)
     const uint32_t nI = ctr->n[cur];
     const unsigned long long tagv = (unsigned long long)tag << 32;
+    long long acc[4] = {0, 0, 0, 0};
     FS_FOR(pos, nI) {
         const uint8_t s = state[pos];
         if (s == FS_STAY) continue;
         const size_t idx = list[pos];
         const Coord c = coord_of(p, idx);
-        if (s == FS_FILLED) {
-            for (int j = 1; j < 19; ++j) {
-                const size_t L = nb_index(p, c, j);
-                if (type[L] != T_GAS) continue;
-                const unsigned long long old = atomicMax(&claim[L], tagv | (unsigned long long)(idx + 1));
-                if (old < tagv) listA[atomicAdd(&ctr->nA, 1u)] = (uint32_t)L;
-            }
-        } else {
-            for (int j = 0; j < 19; ++j) {
-                const size_t L = j == 0 ? idx : nb_index(p, c, j);
-                if (type[L] != T_FLUID) continue;
-                const unsigned long long old = atomicMax(&claim[L], tagv | 1ull);
-                if (old >= tagv) continue;
-                listB[atomicAdd(&ctr->nB, 1u)] = (uint32_t)L;
-                if (p.actPrev) const_cast<uint32_t*>(p.actPrev)[L] = (p.actTag << 2) | 1u;  // was fluid
-                type[L] = T_INTERFACE;
-                link[L] |= LINK_INTERFACE;
-                const double n = to_d(rho[L]);
-                mass[L] = 0.99 * n;
-                exact_add(ctr->acc, 0.01 * n);
-            }
+        // the neighbours' types, then the claims, each loaded together: three round trips instead of one per link.
+        // (A fluid neighbour that another node has turned meanwhile is found by its claim.)
+        const uint8_t want = s == FS_FILLED ? T_GAS : T_FLUID;
+        const unsigned long long mine = tagv | (s == FS_FILLED ? (unsigned long long)(idx + 1) : 1ull);
+        uint8_t tn[19];
+        unsigned long long old[19];
+#pragma unroll
+        for (int j = 0; j < 19; ++j) tn[j] = type[j == 0 ? idx : nb_index(p, c, j)];
+#pragma unroll
+        for (int j = 0; j < 19; ++j) {
+            old[j] = ~0ull;
+            if (tn[j] == want && !(s == FS_FILLED && j == 0)) old[j] = atomicMax(&claim[j == 0 ? idx : nb_index(p, c, j)], mine);
+        }
+        uint32_t first = 0;  // nodes nobody had claimed this step
+#pragma unroll
+        for (int j = 0; j < 19; ++j)
+            if (old[j] < tagv) first |= 1u << j;
+        if (!first) continue;
+        uint32_t at = atomicAdd(s == FS_FILLED ? &ctr->nA : &ctr->nB, (uint32_t)__popc(first));
+        uint32_t* out = s == FS_FILLED ? listA : listB;
+        for (; first; first &= first - 1u) {
+            const int j = __ffs((int)first) - 1;
+            const size_t L = j == 0 ? idx : nb_index(p, c, j);
+            out[at++] = (uint32_t)L;
+            if (s == FS_FILLED) continue;
+            if (p.actPrev) const_cast<uint32_t*>(p.actPrev)[L] = (p.actTag << 2) | 1u;  // was fluid
+            type[L] = T_INTERFACE;
+            link[L] |= LINK_INTERFACE;
+            const double n = to_d(rho[L]);
+            mass[L] = 0.99 * n;
+            exact_local(acc, 0.01 * n);
         }
     }
+    flush_acc(ctr->acc, acc);
 }
 
 // ---- 4. new interface nodes from gas (LB.cpp:1668-1682, node.cpp:26-61) and
@@ -244,6 +306,7 @@ __global__ void __launch_bounds__(FS_BLOCK)
     const uint32_t nI = ctr->n[cur], nA = ctr->nA;
     const uint32_t n = nI > nA ? nI : nA;
     const double rho0 = p.initDensity;
+    long long acc[4] = {0, 0, 0, 0};
     FS_FOR(pos, n) {
         if (pos < nA) {
             const size_t L = listA[pos];
@@ -278,7 +341,7 @@ __global__ void __launch_bounds__(FS_BLOCK)
             uS[L] = u.x; uS[N + L] = u.y; uS[2 * N + L] = u.z;
             hFi[L] = 0.0; hFi[N + L] = 0.0; hFi[2 * N + L] = 0.0;
             if (visc) visc[L] = visc[f];
-            exact_add(ctr->acc, -(0.01 * rho0));
+            exact_local(acc, -(0.01 * rho0));
         }
         if (pos < nI) {
             const uint8_t s = state[pos];
@@ -286,14 +349,15 @@ __global__ void __launch_bounds__(FS_BLOCK)
             const size_t idx = list[pos];
             if ((claim[idx] >> 32) == tag) continue;  // became interface again this step
             if (s == FS_EMPTIED) {
-                exact_add(ctr->acc, mass[idx]);
+                exact_local(acc, mass[idx]);
             } else {
                 const double nn = to_d(rho[idx]);
-                exact_add(ctr->acc, mass[idx] - nn);
+                exact_local(acc, mass[idx] - nn);
                 mass[idx] = nn;
             }
         }
     }
+    flush_acc(ctr->acc, acc);
 }
 
 // Interface candidates after smoothenInterface: unchanged list entries, then the
@@ -321,6 +385,7 @@ __global__ void __launch_bounds__(FS_BLOCK)
                    double* __restrict__ mass, const T* __restrict__ rho, LBKParams p) {
 #pragma clang fp contract(off)
     const uint32_t nI = ctr->n[cur], nA = ctr->nA, nB = ctr->nB;
+    long long acc[4] = {0, 0, 0, 0};
     FS_FOR(q, nI + nA + nB) {
         size_t idx;
         if (!fs_candidate(q, nI, nA, list, state, listA, listB, idx)) continue;
@@ -333,64 +398,108 @@ __global__ void __launch_bounds__(FS_BLOCK)
         for (int j = 1; j < 19; ++j) gasNb = gasNb || tn[j] == T_GAS;
         if (gasNb) continue;
         const double n = to_d(rho[idx]);
-        exact_add(ctr->acc, mass[idx] - n);
+        exact_local(acc, mass[idx] - n);
         mass[idx] = n;
         type[idx] = T_FLUID;
         link[idx] &= ~LINK_INTERFACE;
     }
+    flush_acc(ctr->acc, acc);
+}
+
+// Position of each lane that keeps a value in a list of `count` entries: the workgroup's values stay together and in
+// order, one atomic for all of them. Every lane of the workgroup calls it; n values of this lane.
+__device__ __forceinline__ uint32_t append_at(uint32_t n, uint32_t* count) {
+    __shared__ uint32_t sum[FS_BLOCK / 64], base;
+    const int lane = (int)(threadIdx.x & 63u), wave = (int)(threadIdx.x >> 6);
+    uint32_t incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t v = __shfl_up(incl, off, 64);
+        if (lane >= off) incl += v;
+    }
+    __syncthreads();  // the call before has read sum and base
+    if (lane == 63) sum[wave] = incl;
+    __syncthreads();
+    uint32_t before = 0, all = 0;
+#pragma unroll
+    for (int w = 0; w < FS_BLOCK / 64; ++w) {
+        before += w < wave ? sum[w] : 0u;
+        all += sum[w];
+    }
+    if (threadIdx.x == 0) base = all ? atomicAdd(count, all) : 0u;
+    __syncthreads();
+    return base + before + incl - n;
 }
 
 // ---- 6. removeIsolated, second loop (LB.cpp:1771-1792): no fluid neighbour ->
-// gas; the remaining interface nodes form the next list
+// gas; the remaining interface nodes form the next list. One atomic per workgroup for their places: one per
+// wavefront bound the kernel (262,144 nodes 52 us, now 16) and scattered neighbouring nodes over the list.
 __global__ void __launch_bounds__(FS_BLOCK)
     k_fs_iso_gas(const uint32_t* __restrict__ list, FSCounters* __restrict__ ctr, int cur,
                  const uint8_t* __restrict__ state, const uint32_t* __restrict__ listA,
                  const uint32_t* __restrict__ listB, uint8_t* __restrict__ type, uint32_t* __restrict__ link,
                  const double* __restrict__ mass, uint32_t* __restrict__ next, LBKParams p) {
-    const uint32_t nI = ctr->n[cur], nA = ctr->nA, nB = ctr->nB;
-    FS_FOR(q, nI + nA + nB) {
-        size_t idx;
-        if (!fs_candidate(q, nI, nA, list, state, listA, listB, idx)) continue;
-        if (type[idx] != T_INTERFACE) continue;
-        const Coord c = coord_of(p, idx);
-        uint8_t tn[19];  // all loaded before the test: one round trip
+    const uint32_t nI = ctr->n[cur], nA = ctr->nA, nB = ctr->nB, n = nI + nA + nB;
+    long long acc[4] = {0, 0, 0, 0};
+    for (uint32_t q0 = blockIdx.x * blockDim.x; q0 < n; q0 += gridDim.x * blockDim.x) {
+        const uint32_t q = q0 + threadIdx.x;
+        size_t idx = 0;
+        bool keep = false;
+        if (q < n && fs_candidate(q, nI, nA, list, state, listA, listB, idx) && type[idx] == T_INTERFACE) {
+            const Coord c = coord_of(p, idx);
+            uint8_t tn[19];  // all loaded before the test: one round trip
 #pragma unroll
-        for (int j = 1; j < 19; ++j) tn[j] = type[nb_index(p, c, j)];
-        bool fluidNb = false;
+            for (int j = 1; j < 19; ++j) tn[j] = type[nb_index(p, c, j)];
 #pragma unroll
-        for (int j = 1; j < 19; ++j) fluidNb = fluidNb || tn[j] == T_FLUID;
-        if (fluidNb) {
-            next[atomicAdd(&ctr->n[cur ^ 1], 1u)] = (uint32_t)idx;
-        } else {
-            exact_add(ctr->acc, mass[idx]);
-            type[idx] = T_GAS;
-            link[idx] = 0u;
+            for (int j = 1; j < 19; ++j) keep = keep || tn[j] == T_FLUID;
+            if (!keep) {
+                exact_local(acc, mass[idx]);
+                type[idx] = T_GAS;
+                link[idx] = 0u;
+            }
         }
+        const uint32_t at = append_at(keep ? 1u : 0u, &ctr->n[cur ^ 1]);
+        if (keep) next[at] = (uint32_t)idx;
     }
+    flush_acc(ctr->acc, acc);
 }
 
 // ---- 7. redistributeMass (LB.cpp:1796-1804)
 __global__ void __launch_bounds__(FS_BLOCK)
-    k_fs_redistribute(const uint32_t* __restrict__ next, const FSCounters* __restrict__ ctr, int cur,
+    k_fs_redistribute(const uint32_t* __restrict__ next, FSCounters* __restrict__ ctr, int cur,
                       double* __restrict__ mass) {
 #pragma clang fp contract(off)
     const uint32_t n = ctr->n[cur ^ 1];
+    if (blockIdx.x == 0 && threadIdx.x == 0) ctr->nA = 0;  // k_fs_build_list may count with it
     if (n == 0) return;
     const double add = exact_value(ctr->acc) / (double)n;
     FS_FOR(q, n) mass[next[q]] += add;
 }
 
-// ---- initial interface list
-__global__ void k_fs_build_list(const uint8_t* __restrict__ type, uint32_t* __restrict__ list,
-                                FSCounters* __restrict__ ctr, int cur, size_t N) {
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < N; i += (size_t)gridDim.x * blockDim.x) {
-        const bool it = type[i] == T_INTERFACE;
-        const unsigned long long b = __ballot(it);
-        const int lane = threadIdx.x & 63;
-        uint32_t base = 0;
-        if (lane == 0 && b) base = atomicAdd(&ctr->n[cur], (uint32_t)__popcll(b));
-        base = __shfl(base, 0, 64);
-        if (it) list[base + __popcll(b & ((1ull << lane) - 1ull))] = (uint32_t)i;
+// ---- interface list in lattice order (4,096 nodes of a workgroup stay together): at the start, and every
+// SORT_STEPS passes, since the passes append new nodes and deal the workgroups' parts out in any order, after which
+// neighbouring lanes of k_fs_mass read lines far apart. 16 node types per lane; read-bound. `count` starts at zero
+// and ends as the list's length.
+constexpr int BUILD_NODES = 16;
+__global__ void __launch_bounds__(FS_BLOCK) k_fs_build_list(const uint8_t* __restrict__ type, uint32_t* __restrict__ list,
+                                                            uint32_t* __restrict__ count, size_t N) {
+    const size_t per = (size_t)FS_BLOCK * BUILD_NODES;
+    for (size_t i0 = blockIdx.x * per; i0 < N; i0 += gridDim.x * per) {
+        const size_t i = i0 + threadIdx.x * (size_t)BUILD_NODES;
+        uint32_t itf = 0;  // bit k: node i + k
+        if (i + BUILD_NODES <= N) {
+            const uint4 t = *reinterpret_cast<const uint4*>(type + i);  // type is aligned, i a multiple of 16
+            const uint32_t w[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+            for (int k = 0; k < BUILD_NODES; ++k)
+                if (((w[k / 4] >> (8 * (k % 4))) & 0xFFu) == (uint32_t)T_INTERFACE) itf |= 1u << k;
+        } else {
+            for (size_t k = i; k < N; ++k)
+                if (type[k] == T_INTERFACE) itf |= 1u << (k - i);
+        }
+        if (!__syncthreads_or(itf != 0u)) continue;
+        uint32_t at = append_at((uint32_t)__popc(itf), count);
+        for (; itf; itf &= itf - 1u) list[at++] = (uint32_t)(i + (size_t)(__ffs((int)itf) - 1));
     }
 }
 
@@ -538,19 +647,27 @@ void launch_fs_curved_extra(Prec prec, const void* fpost, const uint32_t* link, 
     k_fs_add_extra<<<1, FS_BLOCK, 0, s>>>(b.list[cur], b.ctr, cur, b.mass);
 }
 
-void launch_fs_build_list(const uint8_t* type, FSBuffers& b, int cur, const LBKParams& p, hipStream_t s) {
-    const size_t N = (size_t)p.X * p.Y * p.Z;
-    size_t g = (N + 255) / 256;
+static void build_list(const uint8_t* type, uint32_t* list, uint32_t* count, const LBKParams& p, hipStream_t s) {
+    const size_t N = (size_t)p.X * p.Y * p.Z, per = (size_t)FS_BLOCK * BUILD_NODES;
+    size_t g = (N + per - 1) / per;
     if (g > 4096) g = 4096;
-    k_fs_build_list<<<(unsigned)g, 256, 0, s>>>(type, b.list[cur], b.ctr, cur, N);
+    k_fs_build_list<<<(unsigned)g, FS_BLOCK, 0, s>>>(type, list, count, N);
+}
+
+void launch_fs_build_list(const uint8_t* type, FSBuffers& b, int cur, const LBKParams& p, hipStream_t s) {
+    build_list(type, b.list[cur], &b.ctr->n[cur], p, s);
 }
 
 template <typename T, bool SHIFT>
 static void fs_step_t(const T* fpost, T* fout, uint8_t* type, uint32_t* link, uint32_t* slipw, double* visc, FSBuffers& b,
                       int cur, int rcur, uint32_t tag, const double* Fnew, bool pull, const LBKParams& p, hipStream_t s) {
     const T* rho = (const T*)b.rho[rcur];
-    k_fs_mass<T, SHIFT><<<FS_GRID, FS_BLOCK, 0, s>>>(fpost, fout, type, b.mass, rho, b.uS, b.list[cur], b.ctr, cur,
-                                                    b.mnew, b.state, p, pull ? 1 : 0);
+    if (pull && !p.slipw && !p.curvw)
+        k_fs_mass<T, SHIFT, true><<<MASS_GRID, MASS_BLOCK, 0, s>>>(fpost, fout, type, b.mass, rho, b.uS, b.list[cur], b.ctr,
+                                                               cur, b.mnew, b.state, p, 1);
+    else
+        k_fs_mass<T, SHIFT, false><<<MASS_GRID, MASS_BLOCK, 0, s>>>(fpost, fout, type, b.mass, rho, b.uS, b.list[cur], b.ctr,
+                                                                cur, b.mnew, b.state, p, pull ? 1 : 0);
     k_fs_apply<<<FS_GRID, FS_BLOCK, 0, s>>>(b.list[cur], b.ctr, cur, b.mnew, b.state, b.mass, type, link);
     k_fs_spread<T><<<FS_GRID, FS_BLOCK, 0, s>>>(b.list[cur], b.ctr, cur, b.state, type, link, b.claim, b.listA, b.listB,
                                                b.mass, rho, tag, p);
@@ -562,6 +679,7 @@ static void fs_step_t(const T* fpost, T* fout, uint8_t* type, uint32_t* link, ui
     k_fs_iso_gas<<<FS_GRID, FS_BLOCK, 0, s>>>(b.list[cur], b.ctr, cur, b.state, b.listA, b.listB, type, link, b.mass,
                                              b.list[cur ^ 1], p);
     k_fs_redistribute<<<FS_GRID, FS_BLOCK, 0, s>>>(b.list[cur ^ 1], b.ctr, cur, b.mass);
+    if (tag % SORT_STEPS == 0) build_list(type, b.list[cur ^ 1], &b.ctr->nA, p, s);
 }
 
 void launch_fs_step(Prec prec, const void* fpost, void* fout, uint8_t* type, uint32_t* link, uint32_t* slipw,
