@@ -1066,6 +1066,7 @@ static int lb_alloc(hyb_lb* l, int slotCap) {
             (rc = ralloc(A, R, "mnew", &b.mnew, N)) || (rc = ralloc(A, R, "state", &b.state, N)) ||
             (rc = ralloc(A, R, "ctr", &b.ctr, 1)))
             return rc;
+        b.actPrev = nullptr;  // of an earlier initialisation; cylinders get theirs in hyb_lb_init
         if (l->hasSlip() && (rc = ralloc(A, R, "actPrev", &b.actPrev, N))) return rc;
     }
     l->slotCap = slotCap;
