@@ -2,7 +2,8 @@
 // inputs unpacked into planes). Bound by the copy to or from pageable host memory that follows (10 to 17 GB/s with
 // the pages' first touch; the kernels move the same bytes at HBM rate). Packing on the host read every plane back
 // and went through them with a stride per node. Before and after, 256^3 nodes: velocity 296 -> 38 ms, density
-// 273 -> 13, types 38 -> 1.5, populations 522 -> 253; 128^3 nodes: populations in 80 -> 12, a force field 3 to 7 -> 1.1;
+// 273 -> 13, types 38 -> 1.5, populations 522 -> 253 (velocity 25, with the
+// pages of the caller's buffer made present meanwhile); 128^3 nodes: populations in 80 -> 12, a force field 3 to 7 -> 1.1;
 // 7,728 elements: e_x 2 -> 0.1 ms.
 //
 // One thread per output value, so the wide side of every access is coalesced: consecutive threads write

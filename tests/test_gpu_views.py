@@ -53,3 +53,25 @@ def test_populations_and_forces_over_several_ranges(precision, size):
     assert np.abs(u[free] - 0.5 * F[free].astype(np.float64)).max() <= tol
     assert np.isnan(u[~act]).all()
     sim.close()
+
+
+def test_views_into_unaligned_buffers():
+    """A large view (whose pages are made present beforehand) writes its own bytes only, wherever the buffer starts."""
+    import ctypes as C
+
+    from hybird_amd import runtime
+    size = (97, 83, 71)
+    sim = _sim(size, "FP64")
+    want = sim.get("u")
+    n = want.nbytes
+    assert n > 8 << 20
+    for shift in (8, 4096 - 8, 4096):
+        print(f"[gpu views] unaligned by {shift}", flush=True)
+        raw = np.full(n + 3 * 4096, 0xA5, dtype=np.uint8)
+        off = -raw.ctypes.data % 4096 + shift
+        need = C.c_size_t(0)
+        rc = runtime.load().hyb_lb_get(sim._lb, b"u", raw.ctypes.data + off, n, C.byref(need))
+        assert rc == 0 and need.value == n
+        assert np.array_equal(raw[off:off + n], want.reshape(-1).view(np.uint8))
+        assert (raw[:off] == 0xA5).all() and (raw[off + n:] == 0xA5).all()
+    sim.close()
