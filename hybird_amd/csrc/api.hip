@@ -327,8 +327,6 @@ struct hyb_lb {
     unsigned long long* dcount = nullptr;
     CoupleRec* cp = nullptr;
     CoupleRecF* cpf = nullptr;
-    NodeBox* boxes = nullptr;
-    int* nslots = nullptr;  // [0] slots this step, [1] boxes marked last step
     int slotCap = 0;
     uint32_t ctag = 0;       // coupling-step tag of the node ownership words
     hyb_dem* dem = nullptr;  // DEM handle coupled at init (read by the host views)
@@ -1095,8 +1093,7 @@ static int lb_alloc(hyb_lb* l, int slotCap) {
     R.push_back(Blk{"f1", l->f[1], pb});
     if ((rc = ralloc(A, R, "type", &l->type, N)) || (rc = ralloc(A, R, "link", &l->link, N)) ||
         (rc = ralloc(A, R, "solid", &l->solid, N)) ||
-        (rc = dalloc(A, &l->maxXYZ, 3 * (size_t)l->Z)) || (rc = dalloc(A, &l->dcount, (size_t)l->Z + 2)) ||
-        (rc = dalloc(A, &l->nslots, 2)))
+        (rc = dalloc(A, &l->maxXYZ, 3 * (size_t)l->Z)) || (rc = dalloc(A, &l->dcount, (size_t)l->Z + 2)))
         return rc;
     if (l->varVisc() && (rc = ralloc(A, R, "visc", &l->visc, N))) return rc;
     if (l->hasSlip() && (rc = ralloc(A, R, "slipw", &l->slipw, N))) return rc;
@@ -1118,7 +1115,7 @@ static int lb_alloc(hyb_lb* l, int slotCap) {
     }
     l->slotCap = slotCap;
     if (slotCap > 0) {
-        if ((rc = dalloc(A, &l->cp, slotCap)) || (rc = dalloc(A, &l->cpf, slotCap)) || (rc = dalloc(A, &l->boxes, slotCap)) ||
+        if ((rc = dalloc(A, &l->cp, slotCap)) || (rc = dalloc(A, &l->cpf, slotCap)) ||
             (rc = dalloc(A, &l->segs, (size_t)slotCap * l->segCap)) || (rc = dalloc(A, &l->segCount, slotCap)))
             return rc;
         HIPCHK(hipMemset(l->segCount, 0, sizeof(uint32_t) * (size_t)slotCap));
@@ -1134,11 +1131,12 @@ static void lb_couple_launch(hyb_lb* l, hyb_dem* d) {
         l->ctag = 1;
     }
     const LBKParams p = l->params();
-    launch_dem_couple_table(d->p, d->b, l->cp, l->cpf, l->nslots, l->unit, l->stream);
+    const DEMBuffers& b = d->b;
+    const CoupleSource src{b.el, d->p.clumps ? b.pelem : nullptr, b.pcor, b.ghostIndex, b.ghostVec, &b.st->nSlots,
+                           d->p.E, d->p.P, l->unit};
     // without free surface no inactive node becomes active and the ownership of an inactive node is never
     // read (views mask it), so every node inside a sphere is marked without reading its link word
-    launch_classify_set(l->nslots, l->slotCap, l->cp, l->boxes, l->nslots + 1, l->solid,
-                        l->freeSurface ? l->link : nullptr, p, l->stream);
+    launch_couple(src, l->slotCap, l->cp, l->cpf, l->solid, l->freeSurface ? l->link : nullptr, p, l->stream);
 }
 
 int hyb_lb_init(hyb_lb* l, hyb_dem* d) {  // LB.cpp:190-219
@@ -1247,7 +1245,6 @@ int hyb_lb_init(hyb_lb* l, hyb_dem* d) {  // LB.cpp:190-219
     launch_lb_init_pops(l->prec, l->f[0], l->link, l->maxXYZ, l->visc, l->initVelocity, l->lbF,
                         l->freeSurface ? l->fsb.rho[0] : nullptr, l->fsb.mass, l->fsb.uS, p, s);
     launch_fill_u32(l->solid, 0u, l->N, s);
-    HIPCHK(hipMemsetAsync(l->nslots, 0, 2 * sizeof(int), s));
     HIPCHK(hipMemsetAsync(l->dcount, 0, sizeof(unsigned long long) * (l->Z + 2), s));
     launch_count_active(l->link, l->dcount, p, s);
     // particle nodes at init (LB.cpp:475-495)

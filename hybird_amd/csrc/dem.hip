@@ -922,52 +922,6 @@ __device__ __forceinline__ double gather_elem(const DEMParams& p, const DEMBuffe
     return xc[1].norm2();
 }
 
-// Coupling records of every particle slot after the DEM step: corrected
-// position and radiusVec (ghosts: origin + period vector with the origin's
-// radiusVec, elmt.cpp:292-298), the element's velocity and angular velocity,
-// radius.
-__global__ void k_dem_couple_table(DEMParams p, DEMBuffers b, CoupleRec* __restrict__ cp, CoupleRecF* __restrict__ cpf,
-                                   int* __restrict__ nslots, Units u) {
-#pragma clang fp contract(off)
-    const El E{b.el, p.E};
-    const int S = b.st->nSlots;
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s == 0) *nslots = S;
-    if (s >= S) return;
-    const int o = s < p.P ? s : (int)b.ghostIndex[s - p.P];  // standard particle
-    const int e = part_elem(p, b, o);
-    V3 x0, rv(0.0, 0.0, 0.0);
-    if (p.clumps) {
-        const double* c = b.pcor + 9 * (size_t)o;
-        x0 = V3(c[0], c[1], c[2]);
-        rv = V3(c[6], c[7], c[8]);
-    } else {
-        x0 = E.v3(EF_X, o);
-    }
-    if (s >= p.P) {
-        const int g = s - p.P;
-        x0 = x0 + V3(b.ghostVec[3 * g], b.ghostVec[3 * g + 1], b.ghostVec[3 * g + 2]);
-    }
-    CoupleRec r;
-    r.x0[0] = x0.x; r.x0[1] = x0.y; r.x0[2] = x0.z;
-    r.rv[0] = rv.x; r.rv[1] = rv.y; r.rv[2] = rv.z;
-    const V3 v = E.v3(EF_X + 3, e), w = E.v3(EF_WG, e);
-    r.v[0] = v.x; r.v[1] = v.y; r.v[2] = v.z;
-    r.w[0] = w.x; r.w[1] = w.y; r.w[2] = w.z;
-    r.r = E.at(EF_RAD, e);
-    r.elem = e;
-    r.pad = 0;
-    cp[s] = r;
-    CoupleRecF q;
-    const V3 cc = x0 / u.Length - rv / u.Length;  // radius = node - cc (LB.cpp:1875)
-    const V3 vs = v / u.Speed, ws = w / u.AngVel;
-    q.c[0] = (float)cc.x; q.c[1] = (float)cc.y; q.c[2] = (float)cc.z;
-    q.v[0] = (float)vs.x; q.v[1] = (float)vs.y; q.v[2] = (float)vs.z;
-    q.w[0] = (float)ws.x; q.w[1] = (float)ws.y; q.w[2] = (float)ws.z;
-    q.pad[0] = q.pad[1] = q.pad[2] = 0.0f;
-    cpf[s] = q;
-}
-
 // Element hydrodynamic force and torque (LB.cpp:1897-1918): the run sums the
 // collision appended for the slots of the element's particles and their ghosts,
 // added exactly (fixed point, so the result does not depend on the order of the
@@ -1172,12 +1126,6 @@ void launch_dem_gather(const DEMParams& p, const DEMBuffers& b, hipStream_t s) {
 }
 
 
-
-void launch_dem_couple_table(const DEMParams& p, const DEMBuffers& b, CoupleRec* cp, CoupleRecF* cpf, int* nslots,
-                             const Units& u, hipStream_t s) {
-    const int cap = p.P + p.Gcap;
-    k_dem_couple_table<<<(cap + 255) / 256 > 0 ? (cap + 255) / 256 : 1, 256, 0, s>>>(p, b, cp, cpf, nslots, u);
-}
 
 void launch_dem_hydro_combine(const DEMParams& p, const DEMBuffers& b, const HydroSink& hs, const Units& u,
                               hipStream_t s) {

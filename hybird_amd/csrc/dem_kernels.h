@@ -223,8 +223,6 @@ void launch_dem_predict(const DEMParams& p, const DEMBuffers& b, hipStream_t s);
 // element's corrected and predicted state (multi-sphere elements only).
 void launch_dem_particles(const DEMParams& p, const DEMBuffers& b, hipStream_t s);
 void launch_dem_energy(const DEMParams& p, const DEMBuffers& b, const double demSize[3], double* out, hipStream_t s);
-void launch_dem_couple_table(const DEMParams& p, const DEMBuffers& b, CoupleRec* cp, CoupleRecF* cpf, int* nslots,
-                             const Units& u, hipStream_t s);
 // FHydro, MHydro and fluidVolume of every element from the run sums of its own
 // and its ghosts' slots (hs: filled by the fused collision, emptied here).
 void launch_dem_hydro_combine(const DEMParams& p, const DEMBuffers& b, const HydroSink& hs, const Units& u,

@@ -16,6 +16,7 @@
 
 #include "common.h"
 #include "hybird_amd.h"
+#include "dem_kernels.h"
 #include "fs_kernels.h"
 #include "lattice.h"
 #include "lb_kernels.h"
@@ -864,6 +865,10 @@ __global__ void k_count_mass(const uint32_t* __restrict__ link, const uint32_t* 
 // (link == nullptr: every node inside, active or not).
 // Where spheres overlap the highest slot index wins, as in the full re-test of
 // LB.cpp:475-495.
+struct NodeBox {  // inclusive bounds
+    int lo[3];
+    int hi[3];
+};
 __device__ __forceinline__ NodeBox slot_box(const CoupleRec& r, const LBKParams& p) {
     const double c[3] = {r.x0[0] / p.unitLength, r.x0[1] / p.unitLength, r.x0[2] / p.unitLength};
     const double rad = r.r / p.unitLength;
@@ -975,24 +980,81 @@ __device__ __forceinline__ void for_slot_batches(const NodeBox& b, int lane, Slo
     }
 }
 
-__global__ void __launch_bounds__(256) k_classify_set(const int* __restrict__ nslots_p, const CoupleRec* __restrict__ cp,
-                               NodeBox* __restrict__ boxes, int* __restrict__ nboxes, uint32_t* __restrict__ solid,
-                               const uint32_t* __restrict__ link, LBKParams p) {
+// Record of particle slot s: a standard particle, or a ghost at its origin plus the period vector (elmt.cpp:277-298).
+// WHOLE: also what the classification does not need (velocities).
+template <bool WHOLE>
+__device__ __forceinline__ CoupleRec slot_record(const CoupleSource& src, int s) {
+#pragma clang fp contract(off)
+    const auto v3 = [&](int f, int e) {
+        const double* a = src.el + (size_t)f * src.E + e;
+        return V3(a[0], a[src.E], a[2 * (size_t)src.E]);
+    };
+    const int o = s < src.P ? s : (int)src.ghostIndex[s - src.P];
+    const int e = src.pelem ? src.pelem[o] : o;
+    V3 x0, rv(0.0, 0.0, 0.0);
+    if (src.pelem) {
+        const double* c = src.pcor + 9 * (size_t)o;
+        x0 = V3(c[0], c[1], c[2]);
+        rv = V3(c[6], c[7], c[8]);
+    } else {
+        x0 = v3(EF_X, o);
+    }
+    if (s >= src.P) {
+        const double* g = src.ghostVec + 3 * (size_t)(s - src.P);
+        x0 = x0 + V3(g[0], g[1], g[2]);
+    }
+    CoupleRec r{};
+    r.x0[0] = x0.x; r.x0[1] = x0.y; r.x0[2] = x0.z;
+    r.rv[0] = rv.x; r.rv[1] = rv.y; r.rv[2] = rv.z;
+    r.r = src.el[(size_t)EF_RAD * src.E + e];
+    r.elem = e;
+    if (WHOLE) {
+        const V3 v = v3(EF_X + 3, e), w = v3(EF_WG, e);
+        r.v[0] = v.x; r.v[1] = v.y; r.v[2] = v.z;
+        r.w[0] = w.x; r.w[1] = w.y; r.w[2] = w.z;
+    }
+    return r;
+}
+__device__ __forceinline__ CoupleRecF scaled_record(const CoupleRec& r, const Units& u) {
+#pragma clang fp contract(off)
+    const V3 x0(r.x0[0], r.x0[1], r.x0[2]), rv(r.rv[0], r.rv[1], r.rv[2]);
+    const V3 cc = x0 / u.Length - rv / u.Length;  // radius = node - cc (LB.cpp:1875)
+    const V3 vs = V3(r.v[0], r.v[1], r.v[2]) / u.Speed, ws = V3(r.w[0], r.w[1], r.w[2]) / u.AngVel;
+    CoupleRecF q;
+    q.c[0] = (float)cc.x; q.c[1] = (float)cc.y; q.c[2] = (float)cc.z;
+    q.v[0] = (float)vs.x; q.v[1] = (float)vs.y; q.v[2] = (float)vs.z;
+    q.w[0] = (float)ws.x; q.w[1] = (float)ws.y; q.w[2] = (float)ws.z;
+    q.pad[0] = q.pad[1] = q.pad[2] = 0.0f;
+    return q;
+}
+
+// Coupling of one step: the slot records for the collision, and the classification; bound by the latency of its
+// dependent loads. Every wavefront makes its slot's record itself (wave-uniform loads that its neighbours share):
+// a kernel of its own for the records took 4.8 us and the gap between two launches, this one 1 us more with 100
+// spheres and 3 us more with 7,728 than with records at hand. A coupled cycle of 64^3 nodes 124.0 -> 121.6 us, of
+// 150 x 97 x 83 233 -> 230.
+__global__ void __launch_bounds__(256) k_couple(CoupleSource src, CoupleRec* __restrict__ cp, CoupleRecF* __restrict__ cpf,
+                                                uint32_t* __restrict__ solid, const uint32_t* __restrict__ link,
+                                                LBKParams p) {
 #pragma clang fp contract(off)
     __shared__ SlotRows shr[SLOT_WAVES];
-    const int ns = *nslots_p;
-    if (blockIdx.x == 0 && threadIdx.x == 0) *nboxes = ns;
+    const int ns = *src.nSlots;
     const int lane = (int)(threadIdx.x & 63);
-    const int unit = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
-    const int nunits = (int)((gridDim.x * blockDim.x) >> 6);
-    SlotRows& sh = shr[threadIdx.x >> 6];
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int unit = (int)blockIdx.x * SLOT_WAVES + wave;
+    const int nunits = (int)gridDim.x * SLOT_WAVES;
+    SlotRows& sh = shr[wave];
     // CLASSIFY_PARTS wavefronts per slot, each on its own 64-row batches of the slot's box, so that the
     // longest chain of one wavefront is one batch (the marks are an order-free maximum)
     for (int us = unit; us < ns * CLASSIFY_PARTS; us += nunits) {
         const int s = us / CLASSIFY_PARTS, part = us % CLASSIFY_PARTS;
-        const CoupleRec r = cp[s];
+        const CoupleRec r = slot_record<false>(src, s);
+        if (part == CLASSIFY_PARTS - 1 && lane == 0) {  // the part with the fewest rows
+            const CoupleRec w = slot_record<true>(src, s);
+            cp[s] = w;
+            cpf[s] = scaled_record(w, src.unit);
+        }
         const NodeBox b = slot_box(r, p);
-        if (lane == 0 && part == 0) boxes[s] = b;
         const V3 cen(r.x0[0] / p.unitLength, r.x0[1] / p.unitLength, r.x0[2] / p.unitLength);
         const double rad = r.r / p.unitLength;
         const uint32_t val = (p.ctag << SOLID_SLOT_BITS) | (uint32_t)(s + 1);
@@ -1257,14 +1319,13 @@ void launch_lb_init_pops(Prec prec, void* f, const uint32_t* link, const int* mx
                                                  Finit[2], (float*)rho, mass, uS);
 }
 
-void launch_classify_set(const int* nslots, int max_slots, const CoupleRec* cp, NodeBox* boxes, int* nboxes,
-                         uint32_t* solid, const uint32_t* link, const LBKParams& p, hipStream_t s) {
+void launch_couple(const CoupleSource& src, int max_slots, CoupleRec* cp, CoupleRecF* cpf, uint32_t* solid,
+                   const uint32_t* link, const LBKParams& p, hipStream_t s) {
     if (max_slots <= 0) return;
     int grid = (max_slots * CLASSIFY_PARTS + SLOT_WAVES - 1) / SLOT_WAVES;  // CLASSIFY_PARTS wavefronts per slot
     if (grid > 16384) grid = 16384;
-    k_classify_set<<<grid, 64 * SLOT_WAVES, 0, s>>>(nslots, cp, boxes, nboxes, solid, link, p);
+    k_couple<<<grid, 64 * SLOT_WAVES, 0, s>>>(src, cp, cpf, solid, link, p);
 }
-
 
 void launch_fill_u32(uint32_t* a, uint32_t v, size_t n, hipStream_t s) {
     if (!n) return;

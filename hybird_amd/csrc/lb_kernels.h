@@ -80,10 +80,16 @@ struct CoupleRecF {
     float pad[3];
 };
 
-// Box of lattice nodes a particle slot may cover (inclusive bounds).
-struct NodeBox {
-    int lo[3];
-    int hi[3];
+// Where the records of the particle slots come from: the element state, and for ghosts their origin and vector.
+struct CoupleSource {
+    const double* el;  // [field][E] (dem_kernels.h)
+    const int* pelem;  // element of each standard particle (nullptr: single spheres, element = particle)
+    const double* pcor;
+    const uint32_t* ghostIndex;
+    const double* ghostVec;
+    const int* nSlots;
+    int E, P;
+    Units unit;
 };
 
 // Hydrodynamic sums of one particle slot over one run of its nodes: a
@@ -154,10 +160,11 @@ void launch_lb_max_active(const uint32_t* link, int* maxXYZ, const LBKParams& p,
 // With free surface, also the initial density (rho), interface mass and interface velocity.
 void launch_lb_init_pops(Prec prec, void* f, const uint32_t* link, const int* maxXYZ, double* visc, const double* u0,
                          const double* Finit, void* rho, double* mass, double* uS, const LBKParams& p, hipStream_t s);
+// The record of every particle slot (cp, cpf), and its nodes marked in solid.
 // link == nullptr: mark every node inside a sphere, active or not (for lattices whose
 // inactive nodes stay inactive and are never read as particle nodes)
-void launch_classify_set(const int* nslots, int max_slots, const CoupleRec* cp, NodeBox* boxes, int* nboxes,
-                         uint32_t* solid, const uint32_t* link, const LBKParams& p, hipStream_t s);
+void launch_couple(const CoupleSource& src, int max_slots, CoupleRec* cp, CoupleRecF* cpf, uint32_t* solid,
+                   const uint32_t* link, const LBKParams& p, hipStream_t s);
 // Non-temporal device copy of `bytes` with 4-, 8- or 16-byte accesses per lane
 // (false: unsupported width).
 bool launch_copy_probe(int width, const void* src, void* dst, size_t bytes, hipStream_t s);
