@@ -26,7 +26,8 @@
 //
 // Data that crosses workgroups between two fences (the exchange records, the barrier words) is read and written
 // with device-scope atomics only. All workgroups must be resident at once: dem_run_fits compares their number
-// with what the device holds, and larger beds use the per-launch kernels. A barrier that does not complete within
+// with what the device holds, and larger beds use the per-launch kernels. Two such launches of one process cannot
+// wait for each other: all handles use one stream. A barrier that does not complete within
 // BARRIER_SECONDS (other processes holding the device) ends the launch with DEM_ERR_BARRIER.
 #include <hip/hip_runtime.h>
 
