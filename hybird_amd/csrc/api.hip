@@ -1078,16 +1078,36 @@ int hyb_lb_create(const hyb_config* cfg, hyb_lb** out) {  // LB.cpp:85-188 + LB.
     return HYB_OK;
 }
 
+// Gives a handle's slabs back, with every pointer into them: an initialisation sets only those its configuration and
+// DEM handle need, and those decide which kernels run (curved walls, slip walls, free surface).
+static void lb_release(hyb_lb* l) {
+    l->saved.clear();
+    l->arena.release();
+    l->f[0] = l->f[1] = nullptr;
+    l->type = nullptr;
+    l->link = l->slipw = l->curvw = l->solid = nullptr;
+    l->macBuf[0] = l->macBuf[1] = nullptr;
+    l->macCur = 0;
+    l->segs = nullptr;
+    l->segCount = nullptr;
+    l->visc = nullptr;
+    l->maxXYZ = nullptr;
+    l->dcount = nullptr;
+    l->cp = nullptr;
+    l->cpf = nullptr;
+    l->slotCap = 0;
+    l->fsb = FSBuffers{};
+}
+
 static int lb_alloc(hyb_lb* l, int slotCap) {
     const size_t N = l->N;
     int rc;
     if ((rc = errword_alloc(l->err))) return rc;
     errword_clear(l->err);
     const size_t pb = l->popBytes();
+    lb_release(l);
     std::vector<Blk>& R = l->saved;
-    R.clear();
     Arena& A = l->arena;
-    A.release();
     if ((rc = A.take(&l->f[0], pb)) || (rc = A.take(&l->f[1], pb))) return rc;
     R.push_back(Blk{"f0", l->f[0], pb});
     R.push_back(Blk{"f1", l->f[1], pb});
@@ -1110,7 +1130,6 @@ static int lb_alloc(hyb_lb* l, int slotCap) {
             (rc = ralloc(A, R, "mnew", &b.mnew, N)) || (rc = ralloc(A, R, "state", &b.state, N)) ||
             (rc = ralloc(A, R, "ctr", &b.ctr, 1)))
             return rc;
-        b.actPrev = nullptr;  // of an earlier initialisation; cylinders get theirs in hyb_lb_init
         if (l->hasSlip() && (rc = ralloc(A, R, "actPrev", &b.actPrev, N))) return rc;
     }
     l->slotCap = slotCap;
