@@ -154,7 +154,11 @@ struct Arena {
         if (bytes > left) {
             const size_t size = std::max(bytes, slab);
             void* q = nullptr;
-            HIPCHK(hipMalloc(&q, size));
+            const hipError_t e = hipMalloc(&q, size);
+            if (e != hipSuccess) {
+                (void)hipGetLastError();  // reported here, not again by the next launch on another handle
+                return fail(HYB_E_HIP, std::string("device allocation: ") + hipGetErrorString(e));
+            }
             slabs.push_back(q);
             if (size > slab) {  // the rest of the current slab stays in use
                 *p = q;
@@ -1081,6 +1085,7 @@ int hyb_lb_create(const hyb_config* cfg, hyb_lb** out) {  // LB.cpp:85-188 + LB.
 // Gives a handle's slabs back, with every pointer into them: an initialisation sets only those its configuration and
 // DEM handle need, and those decide which kernels run (curved walls, slip walls, free surface).
 static void lb_release(hyb_lb* l) {
+    l->inited = false;  // until the initialisation that asked for this has succeeded
     l->saved.clear();
     l->arena.release();
     l->f[0] = l->f[1] = nullptr;

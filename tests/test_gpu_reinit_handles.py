@@ -53,3 +53,59 @@ def test_lattice_with_a_cylinder_initialised_again_without_one(precision):
     assert (got[0]["types"] == 3).any()
     for name, v in got[1].items():
         assert np.array_equal(got[0][name], v, equal_nan=v.dtype != np.uint8), name
+
+
+def _bed_of_wide_spheres(L, runtime, conf, lb):
+    """A DEM handle whose run-sum lists no device can hold: 300 spheres, the largest of radius 2,000."""
+    from hybird_amd._abi import element_records
+
+    rng = np.random.default_rng(3)
+    r = np.full(300, 2.0)
+    r[0] = 2000.0
+    rec = element_records(rng.uniform(3.0, 7.0, (300, 3)), r)
+    wide = type(conf)()
+    C.memmove(C.byref(wide), C.byref(conf), C.sizeof(conf))
+    wide.pairCapacity = 50_000
+    dem = C.c_void_p()
+    assert L.hyb_dem_create(C.byref(wide), len(rec), rec.ctypes.data, C.byref(dem)) == 0
+    assert L.hyb_dem_init(dem, lb) == 0
+    return dem
+
+
+def test_lattice_whose_second_initialisation_fails():
+    """The lattice is as before its first initialisation: every call on its state is refused, and it can be
+    initialised again."""
+    from hybird_amd import runtime
+    from hybird_amd._abi import config_from_cfg, element_records
+    from hybird_amd.cfg import base_config
+
+    L = runtime.load()
+    conf = config_from_cfg(base_config(lbSizeX=12, lbSizeY=11, lbSizeZ=13, boundary0=7, boundary1=7, boundary2=7,
+                                       boundary3=7, lbFX=1.0e-5))
+    rec = element_records(np.array([[5.0, 5.0, 6.0]]), np.array([2.2]))
+    sim, new = runtime.Simulation(conf, rec), runtime.Simulation(conf, rec)
+    print("[gpu reinit handles] lattice, second initialisation fails", flush=True)
+    wide = _bed_of_wide_spheres(L, runtime, conf, sim._lb)
+    assert L.hyb_lb_init(sim._lb, wide) == -2  # HYB_E_HIP
+    new.step_lb(1)  # another handle's launch doesn't report the failed allocation again
+    need = C.c_size_t(0)
+    buf = np.zeros(8 * 19 * 12 * 11 * 13, dtype=np.uint8)
+    state = -3  # HYB_E_STATE
+    assert L.hyb_lb_step(sim._lb, sim._dem) == state
+    assert L.hyb_lb_fs_step(sim._lb) == state
+    assert L.hyb_lb_couple(sim._lb, sim._dem, None) == state
+    assert L.hyb_lb_get(sim._lb, b"f", buf.ctypes.data, buf.nbytes, C.byref(need)) == state
+    assert L.hyb_lb_set_force_field(sim._lb, buf.ctypes.data) == state
+    assert L.hyb_lb_set_populations(sim._lb, buf.ctypes.data) == state
+    assert L.hyb_adj_forward(sim._lb, sim._dem, 2, 1) == state
+    assert L.hyb_state_save(sim._lb, None, b"/dev/null") == state
+    assert L.hyb_lb_wall_fhydro_into(sim._lb, buf.ctypes.data, 18) == state
+    assert L.hyb_lb_init(sim._lb, sim._dem) == 0
+    sim.step_lb(3)
+    new.step_lb(2)
+    for name in ("types", "f", "u", "pflag"):
+        v = new.get(name)
+        assert np.array_equal(sim.get(name), v, equal_nan=v.dtype == np.float64), name
+    assert L.hyb_dem_destroy(wide) == 0
+    sim.close()
+    new.close()
