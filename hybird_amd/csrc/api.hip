@@ -583,9 +583,12 @@ static int dem_run_reset(hyb_dem* d) {
     return HYB_OK;
 }
 
+// An initialisation that fails leaves the handle as before its first one: its parameters and buffers are replaced
+// from here on.
 static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
     const LatticeInfo* lb = &lbi;
     const hyb_config& c = d->cfg;
+    d->inited = false;
     d->unit = lb->unit;
     const Units& U = d->unit;
     // DEM.cpp:185-233
@@ -831,6 +834,8 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
     Arena& A = d->arena;
     R.clear();
     A.release();
+    d->view = nullptr;
+    d->wholeStep = false;
     if ((rc = ralloc(A, R, "el", &b.el, el.size())) || (rc = ralloc(A, R, "st", &b.st, 1)) ||
         (rc = ralloc(A, R, "ghostIndex", &b.ghostIndex, p.Gcap)) || (rc = ralloc(A, R, "ghostVec", &b.ghostVec, 3 * (size_t)p.Gcap)) ||
         (rc = ralloc(A, R, "pairs", &b.pairs, 2 * (size_t)p.pairCap)) || (rc = ralloc(A, R, "nearWall", &b.nearWall, std::max(P, 1))) ||
@@ -1336,6 +1341,7 @@ int hyb_lb_couple(hyb_lb* l, hyb_dem* d, int32_t* newNeighborList) {  // LB.cpp:
     // step, so the rebuild handshake flag is consumed unconditionally.
     if (newNeighborList) *newNeighborList = 0;
     if (!d || !d->P) return HYB_OK;
+    if (!d->inited) return fail(HYB_E_STATE, "hyb_lb_couple: DEM handle not initialised");
     lb_couple_launch(l, d);
     HIPCHK(hipGetLastError());
     return HYB_OK;
@@ -1347,6 +1353,7 @@ static int lb_step(hyb_lb* l, hyb_dem* d, bool hydro) {
     if (int rc = lb_pending(l)) return rc;
     const LBKParams p = l->params();
     const bool withParticles = d && d->P && l->slotCap > 0;
+    if (withParticles && !d->inited) return fail(HYB_E_STATE, "hyb_lb_step: DEM handle not initialised");
     hipEvent_t e0 = nullptr, e1 = nullptr;
     if (l->profiling) {
         if (l->evUsed + 2 > l->evs.size()) {

@@ -109,3 +109,38 @@ def test_lattice_whose_second_initialisation_fails():
     assert L.hyb_dem_destroy(wide) == 0
     sim.close()
     new.close()
+
+
+def test_dem_handle_whose_second_initialisation_fails():
+    """Every call on the handle is refused, also from the lattice it is coupled to, and it can be initialised again."""
+    from hybird_amd import runtime
+
+    L = runtime.load()
+    cfg, rec, _ = load_case("drum")
+    conf = fixture_config(cfg)
+    sim, new = runtime.Simulation(conf, rec), runtime.Simulation(conf, rec)
+    print("[gpu reinit handles] DEM handle, second initialisation fails", flush=True)
+    size = (C.c_int32 * 3)(*[int(np.floor(conf.lbSize[k] / conf.unitLength + 0.5)) for k in range(3)])
+    rotating = (C.c_int32 * 6)(*conf.boundary)
+    rotating[2] = 6  # the drum's rotating y walls are not supported
+    init_args = [size, C.c_double(conf.unitLength), C.c_double(1.0e-4), C.c_double(conf.unitDensity), (C.c_double * 3)()]
+    assert L.hyb_dem_init_lattice(sim._dem, rotating, *init_args) == -5  # HYB_E_UNSUPPORTED
+    need = C.c_size_t(0)
+    buf = np.zeros(1 << 20, dtype=np.uint8)
+    state = -3  # HYB_E_STATE
+    assert L.hyb_dem_step(sim._dem) == state
+    assert L.hyb_dem_set_save_count(sim._dem, 1) == state
+    assert L.hyb_dem_get(sim._dem, b"e_x", buf.ctypes.data, buf.nbytes, C.byref(need)) == state
+    assert L.hyb_state_save(None, sim._dem, b"/dev/null") == state
+    assert L.hyb_lb_init(sim._lb, sim._dem) == state
+    assert L.hyb_lb_couple(sim._lb, sim._dem, None) == state
+    assert L.hyb_lb_step(sim._lb, sim._dem) == state
+    assert L.hyb_cycle(sim._lb, sim._dem, 1) == state
+    assert L.hyb_dem_init(sim._dem, sim._lb) == 0 and L.hyb_lb_init(sim._lb, sim._dem) == 0
+    for s in (sim, new):
+        s.cycle(5)
+    for name in ("types", "f", "e_x", "e_forces"):
+        v = new.get(name)
+        assert np.array_equal(sim.get(name), v, equal_nan=v.dtype == np.float64), name
+    sim.close()
+    new.close()
