@@ -282,6 +282,7 @@ struct hyb_dem {
     Arena arena;             // every device buffer below except the saving ones
     std::vector<Blk> saved;  // persistent device state
     double* view = nullptr;  // packed host view [E][24]
+    std::mutex viewLock;     // held from packing a view to the end of its copy (several threads may read one handle)
     // MercuryDPM-format saving (DEM.cpp:355-360, 1131-1146): captures of the
     // saving sub-steps of the last hyb_dem_step, one slot each
     int saveCount = 0;
@@ -374,6 +375,8 @@ struct hyb_lb {
     std::vector<Blk> saved;  // persistent device state
     void* view = nullptr;    // packed part of a host view or input (viewBytes, at most VIEW_BYTES)
     size_t viewBytes = 0;
+    std::mutex viewLock;     // held while `view`, `scratch` or `mac` serves a view or an input (several threads may
+                             // read one handle)
 
     bool varVisc() const { return nonNewtonian || turbulenceOn || frictional; }
     bool hasSlip() const {
@@ -1436,6 +1439,7 @@ static int view_chunks(hyb_lb* l, size_t per, F&& f) {
 
 int hyb_lb_set_force_field(hyb_lb* l, const float* F) {
     if (!l || !l->inited) return fail(HYB_E_STATE, "hyb_lb_set_force_field before init");
+    const std::lock_guard<std::mutex> writing(l->viewLock);
     HIPCHK(hipStreamSynchronize(l->stream));
     if (!F) {
         if (l->ffield) {
@@ -1458,6 +1462,7 @@ int hyb_lb_set_force_field(hyb_lb* l, const float* F) {
 int hyb_lb_set_populations(hyb_lb* l, const double* f) {
     if (!l || !f) return fail(HYB_E_ARG, "hyb_lb_set_populations: null argument");
     if (!l->inited || l->steps != 0) return fail(HYB_E_STATE, "populations can only be set before the first step");
+    const std::lock_guard<std::mutex> writing(l->viewLock);
     HIPCHK(hipStreamSynchronize(l->stream));
     const int rc = view_chunks(l, 19 * 8, [&](size_t i0, size_t i1) -> int {
         HIPCHK(hipMemcpyAsync(l->view, f + 19 * i0, 19 * 8 * (i1 - i0), hipMemcpyHostToDevice, l->stream));
@@ -1771,6 +1776,7 @@ static int mass_view(hyb_lb* l, const std::vector<uint32_t>& lk, std::vector<dou
 int hyb_lb_get(hyb_lb* l, const char* cname, void* host, size_t cap, size_t* need) {
     if (!l || !cname) return fail(HYB_E_ARG, "hyb_lb_get: null argument");
     if (!l->inited) return fail(HYB_E_STATE, "hyb_lb_get before init");
+    const std::lock_guard<std::mutex> reading(l->viewLock);
     HIPCHK(hipStreamSynchronize(l->stream));
     if (int rc = lb_pending(l)) return rc;
     const std::string name(cname);
@@ -2016,6 +2022,7 @@ int hyb_dem_saved_get(hyb_dem* d, int32_t event, const char* cpart, void* host, 
 int hyb_dem_get(hyb_dem* d, const char* cname, void* host, size_t cap, size_t* need) {
     if (!d || !cname) return fail(HYB_E_ARG, "hyb_dem_get: null argument");
     if (!d->inited) return fail(HYB_E_STATE, "hyb_dem_get before init");
+    const std::lock_guard<std::mutex> reading(d->viewLock);
     HIPCHK(hipStreamSynchronize(d->stream));
     const std::string name(cname);
     const int P = d->P, NE = d->E;

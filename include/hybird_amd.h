@@ -206,6 +206,7 @@ int hyb_cycle(hyb_lb* lb, hyb_dem* dem, int32_t n);
  *       summed exactly); "status" f64[3]: max |u|^2 over active nodes, active nodes, active nodes with
  *       viscosity > 0.95 (maxTau - 0.5) / 3 (IO.cpp:835-850, 969-985; free surface: needs capture)
  * *bytes_needed receives the size; nothing is copied when capacity is too small.
+ * Several threads may read one handle while nothing steps it; its views are made one at a time.
  * N = lbSize product; E elements; P particles including ghosts. */
 int hyb_lb_get(hyb_lb* lb, const char* name, void* host, size_t capacity, size_t* bytes_needed);
 int hyb_dem_get(hyb_dem* dem, const char* name, void* host, size_t capacity, size_t* bytes_needed);
