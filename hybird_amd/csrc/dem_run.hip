@@ -34,6 +34,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "dem_barrier.h"
 #define HYB_DEM_POW_ATTR __attribute__((noinline))
 #include "dem_device.h"
 #include "dem_kernels.h"
@@ -43,11 +44,8 @@ namespace hyb {
 
 namespace {
 
-typedef unsigned long long u64;
-
-constexpr u64 SLOT_EMPTY = ~0ull;
-constexpr u64 SLOT_TIMEOUT = ~0ull - 1;  // above every |x1|^2 and every error code
 constexpr u64 BITS_INF = 0x7FF0000000000000ull;
+constexpr u64 TICKS_PER_SECOND = 100000000;  // wall_clock64
 constexpr u64 BARRIER_SECONDS = 20;
 constexpr int ENT_LANE = 8;  // neighbours per lane kept in LDS (4 x 8 per element; more are read from memory)
 constexpr uint32_t NO_GHOST = 0xFFFFFFFFu;
@@ -131,11 +129,18 @@ __device__ __forceinline__ u64 wave_max_last(u64 v) {
     return dpp_max<0x143, 0xC>(v);  // row_bcast:31 into rows 2 and 3
 }
 
+struct DeviceWords {
+    static __device__ __forceinline__ u64 load(u64* w) { return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); }
+    static __device__ __forceinline__ void store(u64* w, u64 v) {
+        __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    static __device__ __forceinline__ u64 now() { return wall_clock64(); }
+    static __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
+};
+
 template <bool ONE>
-struct Grid {
-    u64* slots;  // [3][workgroups]
-    unsigned n;  // barriers passed so far
-    int nwg, waves;
+struct Grid : Meeting<DeviceWords> {
+    int waves;
 
     // Maximum over the whole grid of `mine`; every store before it is visible to the exchange loads after it.
     // FULL: plain stores before it are visible to plain loads after it in every workgroup. Returns
@@ -160,35 +165,18 @@ struct Grid {
             ++n;
             return v;
         } else {
-            u64* set = slots + (size_t)(n % 3u) * nwg;
             if (threadIdx.x == 0) {
                 if constexpr (FULL) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-                __hip_atomic_store(&set[blockIdx.x], v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                arrive((int)blockIdx.x, v);
             }
-            u64 m = 0;
-            for (int i = (int)threadIdx.x; i < nwg; i += (int)blockDim.x) {
-                u64 s = __hip_atomic_load(&set[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (s == SLOT_EMPTY) {
-                    const u64 t0 = wall_clock64();  // 100 MHz
-                    do {
-                        __builtin_amdgcn_s_sleep(1);
-                        s = __hip_atomic_load(&set[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    } while (s == SLOT_EMPTY && wall_clock64() - t0 < BARRIER_SECONDS * 100000000ull);
-                    if (s == SLOT_EMPTY) s = SLOT_TIMEOUT;
-                }
-                m = s > m ? s : m;
-            }
-            m = wave_max_last(m);
+            const u64 m = wave_max_last(wait_all((int)threadIdx.x, (int)blockDim.x, BARRIER_SECONDS * TICKS_PER_SECOND));
             if ((threadIdx.x & 63) == 63) all[wave] = m;
             __syncthreads();
 #pragma unroll
             for (int w = 0; w < W; ++w) v = all[w] > v ? all[w] : v;
-            // everybody has arrived here, hence left the previous barrier: its word is free again
-            if (threadIdx.x == 0)
-                __hip_atomic_store(&slots[(size_t)((n + 2u) % 3u) * nwg + blockIdx.x], SLOT_EMPTY, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-            if constexpr (FULL) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+            if (threadIdx.x == 0) free_last((int)blockIdx.x);
             ++n;
+            if constexpr (FULL) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
             return v;
         }
     }
@@ -686,7 +674,7 @@ __device__ __forceinline__ int rebuild_body(const DEMParams& p, const DEMBuffers
 template <bool SP, bool ONE>
 __device__ __attribute__((noinline)) RebuildResult rebuild_lists(const DEMRunArgs* a, unsigned n, int e, int c, int ilo,
                                                                  int size, double x, double y, double z) {
-    Grid<ONE> grid{a->b.runSlots, n, (int)gridDim.x, (int)(blockDim.x >> 6)};
+    Grid<ONE> grid{{a->b.runSlots, n, (int)gridDim.x}, (int)(blockDim.x >> 6)};
     RebuildResult r;
     r.code = rebuild_body<SP, ONE>(a->p, a->b, grid, e, c, ilo, size, V3(x, y, z));
     r.n = grid.n;
@@ -811,7 +799,7 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
     // quads past the last element repeat it without particles (size 0): they store nothing
     const int size = e0 < p.E ? (CL ? b.efirst[e + 1] - ilo : 1) : 0;
     const bool multi = CL && size > 1;
-    Grid<ONE> grid{b.runSlots, b.st2->barriers, (int)gridDim.x, (int)(blockDim.x >> 6)};
+    Grid<ONE> grid{{b.runSlots, b.st2->barriers, (int)gridDim.x}, (int)(blockDim.x >> 6)};
     u64 vm = *reinterpret_cast<const u64*>(b.vmax);
     double maxDisp = b.st->maxDisp;
     V3 proto;
@@ -1198,10 +1186,11 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
                     for (int q = 0; q < 3; ++q) b.hist[3 * (size_t)en.z + q] = b.entHist[3 * (size_t)j + q];
             }
     }
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        if (err) {
+    if (threadIdx.x == 0) {
+        const Leaving end = leaving((int)blockIdx.x, err);
+        if (end == LEAVE_ERROR) {
             dem_error(p, b, err);
-        } else {
+        } else if (end == LEAVE_STATE) {
             if (!force) {
                 *reinterpret_cast<u64*>(b.vmax) = vm;
                 b.st->maxDisp = maxDisp;
