@@ -80,7 +80,8 @@ class HybConfig(C.Structure):
         ("frictionCoefFluid", C.c_double),
         ("tangentialModel", C.c_int32),
         ("wallContacts", C.c_int32),
-        ("reserved", C.c_int32 * 2),
+        ("demStepWait", C.c_int32),
+        ("reserved", C.c_int32 * 1),
     ]
 
 
@@ -135,6 +136,7 @@ def config_from_cfg(cfg: dict, collision: str = "BGK", precision: str = "FP64", 
     c.fluidMass = float(g("fluidMass", 0.0))
     c.rheology = HYB_RHEOLOGY_FRICTIONAL if str(g("rheology", "BINGHAM")).upper() == "FRICTIONAL" else HYB_RHEOLOGY_BINGHAM
     c.frictionCoefFluid = float(g("frictionCoefFluid", 0.0))
+    c.demStepWait = int(g("demStepWait", 0))
     c.tangentialModel = (HYB_TANGENTIAL_SPRING if str(g("tangentialModel", "VISCOUS")).upper() == "SPRING"
                          else HYB_TANGENTIAL_VISCOUS)
     c.wallContacts = (HYB_WALL_CONTACTS_ALL if str(g("wallContacts", "FIRST")).upper() == "ALL"

@@ -10,6 +10,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <exception>
@@ -237,6 +238,9 @@ void errword_free(ErrWord& w) {
     w.host = w.dev = nullptr;
 }
 
+// The word after it counts steps done by one workgroup.
+unsigned errword_alone(const ErrWord& w) { return w.host ? (unsigned)__atomic_load_n(w.host + 1, __ATOMIC_ACQUIRE) : 0u; }
+
 int errword_code(const ErrWord& w) { return w.host ? __atomic_load_n(w.host, __ATOMIC_ACQUIRE) : 0; }
 
 void errword_clear(ErrWord& w) {
@@ -278,6 +282,8 @@ struct hyb_dem {
     int64_t substeps = 0;
     bool wholeStep = false;  // a DEM step is one launch (launch_dem_run); otherwise three per sub-step
     bool entStale = false;   // the per-element pair entries of that launch do not belong to the current lists
+    unsigned aloneSeen = 0;  // steps done by one workgroup (dem_run.hip) that the host knows of
+    unsigned apart = 0, apartNext = 0;  // steps still to be made with the launches of dem.hip since, and after the next
     ErrWord err;             // device-side failures of the DEM kernels
     Arena arena;             // every device buffer below except the saving ones
     std::vector<Blk> saved;  // persistent device state
@@ -445,8 +451,8 @@ static int dem_pending(const hyb_dem* d) {
         return fail(HYB_E_NUMERIC, "DEM: non-finite element velocity; the DEM stopped at that sub-step");
     return fail(HYB_E_CAPACITY, "DEM device error " + std::to_string(e) +
                                     " (1/4: ghost or pair capacity, 2: particle outside the cell grid, 3: stencil outside"
-                                    " the cell table, 5: more than 16 objects near one particle, 7: the workgroups of a"
-                                    " DEM step did not meet); the DEM stopped at that sub-step");
+                                    " the cell table, 5: more than 16 objects near one particle, 7: a workgroup of a DEM"
+                                    " step stopped coming); the DEM stopped at that sub-step");
 }
 
 static int lb_pending(const hyb_lb* l) {
@@ -579,10 +585,19 @@ int hyb_dem_init_lattice(hyb_dem* d, const int32_t boundary[6], const int32_t lb
     return dem_init(d, li);
 }
 
+// Time the workgroups of a step wait for each other at its start before one of them does the step alone: far above the
+// microseconds a launch takes on a device of its own, and above most kernels of others that it may have to wait for.
+// One workgroup alone takes 40 ms for a step of 20,000 spheres, so a handle that has met this once makes its next
+// STEPS_APART steps with the launches of dem.hip, and twice as many each further time.
+constexpr int STEP_WAIT_NS = 20000000;
+constexpr unsigned STEPS_APART = 256, STEPS_APART_MOST = 1u << 20;
+
 // Barrier words and counter of the whole-step kernel as before its first launch.
 static int dem_run_reset(hyb_dem* d) {
-    HIPCHK(hipMemsetAsync(d->b.runSlots, 0xFF, 24 * (size_t)dem_run_workgroups(d->p), d->stream));
-    HIPCHK(hipMemsetAsync(d->b.st2, 0, sizeof(DEMRunState), d->stream));
+    const size_t wg = (size_t)dem_run_workgroups(d->p);
+    HIPCHK(hipMemsetAsync(d->b.runSlots, 0xFF, 24 * wg, d->stream));
+    HIPCHK(hipMemsetAsync(d->b.runSlots + 3 * wg, 0, 8 * wg, d->stream));
+    HIPCHK(hipMemsetAsync(d->b.st2, 0, offsetof(DEMRunState, alone), d->stream));
     return HYB_OK;
 }
 
@@ -854,15 +869,21 @@ static int dem_init(hyb_dem* d, const LatticeInfo& lbi) {
         (rc = dalloc(A, &b.wcf, (size_t)std::max(P, 1) * wall_slots(p))))
         return rc;
     HIPCHK(hipMemset(b.wcf, 0, sizeof(ContactForce) * (size_t)std::max(P, 1) * wall_slots(p)));
-    d->wholeStep = dem_run_fits(p);
+    // a launch over several workgroups needs them on the device together
+    d->wholeStep = dem_run_fits(p) && (c.demStepWait >= 0 || dem_run_workgroups(p) == 1);
+    p.waitTicks = (unsigned)(c.demStepWait > 0 ? c.demStepWait : STEP_WAIT_NS) / 10u;
+    __atomic_store_n(d->err.host + 1, 0, __ATOMIC_RELEASE);
+    d->aloneSeen = d->apart = 0;
+    d->apartNext = STEPS_APART;
     if (d->wholeStep) {
         const size_t wg = (size_t)dem_run_workgroups(p);
-        if ((rc = dalloc(A, &b.runSlots, 3 * wg)) || (rc = dalloc(A, &b.st2, 1)) || (rc = dalloc(A, &b.runCount, RUN_COUNTS * wg)) ||
+        if ((rc = dalloc(A, &b.runSlots, 4 * wg)) || (rc = dalloc(A, &b.st2, 1)) || (rc = dalloc(A, &b.runCount, RUN_COUNTS * wg)) ||
             (rc = dalloc(A, &b.xch, 2 * RUN_REC * (size_t)P)) || (rc = dalloc(A, &b.pairCount, (size_t)P)) ||
             (rc = dalloc(A, &b.csrTmp, 2 * (size_t)p.pairCap)) || (rc = dalloc(A, &b.ent, 2 * (size_t)p.pairCap)) ||
             (p.spring && (rc = dalloc(A, &b.entHist, 6 * (size_t)p.pairCap))))
             return rc;
         if ((rc = dem_run_reset(d))) return rc;
+        HIPCHK(hipMemsetAsync(&b.st2->alone, 0, sizeof(unsigned), d->stream));
     }
     if (p.allWalls) {
         if ((rc = ralloc(A, R, "nearWallMask", &b.nearWallMask, (size_t)std::max(P, 1)))) return rc;
@@ -970,7 +991,14 @@ int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
     if (!d || !d->inited) return fail(HYB_E_STATE, "hyb_dem_step before hyb_dem_init");
     if (int rc = dem_pending(d)) return rc;
     d->saveEvents.clear();
-    const bool whole = d->wholeStep && !d->saveCount;
+    const unsigned alone = errword_alone(d->err);
+    if (alone != d->aloneSeen) {
+        d->aloneSeen = alone;
+        d->apart = d->apartNext;
+        d->apartNext = std::min(2 * d->apartNext, STEPS_APART_MOST);
+    }
+    const bool whole = d->wholeStep && !d->saveCount && !d->apart;
+    if (d->apart) --d->apart;
     for (int it = 0; it < d->multiStep; ++it) {
         d->demTimeStep++;
         d->demTime += d->deltat;
@@ -2212,6 +2240,10 @@ int hyb_dem_get(hyb_dem* d, const char* cname, void* host, size_t cap, size_t* n
              (double)p.nCells[1], (double)p.nCells[2], d->demTime, (double)d->demTimeStep, d->deltat, (double)d->multiStep,
              (double)P, d->dampCoeff, d->knConst, d->ksConst, (double)st.newNeighborList};
         return put(v.data(), v.size() * 8, host, cap, need);
+    }
+    if (name == "alone_steps") {
+        const double n = errword_alone(d->err);
+        return put(&n, 8, host, cap, need);
     }
     if (name == "rebuilds") {
         const double r = st.rebuilds;

@@ -5,7 +5,16 @@
 // knows that all have arrived and the maximum of their values. Three sets of words rotate: a set is empty again
 // before it comes next, since nobody reaches meeting n + 1 before everybody has left meeting n - 1.
 //
-// M: the memory of the words, with load, store, now (in ticks) and pause.
+// A launch begins with a roll call, since nothing promises that its workgroups are on the device together: another
+// process's work, or a mask, may leave too few CUs, and two such launches of two processes can each hold a part and
+// wait for the other. Each workgroup has one more word, 2 g after g launches, and checks in as it starts: 2 g + 2. At
+// the first meeting, a workgroup that has waited long enough for another refuses it, by making that word 2 g + 1,
+// unless the other has checked in and is only on its way. A word changes once, so the launch meets if all have checked
+// in, and otherwise nobody sees everybody arrive: one that was refused says so when it comes. Then all leave, and the
+// last to leave does the work alone. Checking in so early takes it out of the way of the first meeting.
+//
+// M: the memory of the words, with load, store, swap (compare and swap; the old value), add (the old value), now (in
+// ticks) and pause.
 #pragma once
 
 namespace hyb {
@@ -14,10 +23,11 @@ typedef unsigned long long u64;
 
 constexpr u64 SLOT_EMPTY = ~0ull;
 constexpr u64 SLOT_TIMEOUT = ~0ull - 1;  // above every value
+constexpr u64 SLOT_PRESENT = 0, SLOT_REFUSED = 1;  // verdicts of the roll call
 
 template <class M>
 struct Meeting {
-    u64* slots;  // [3][workgroups]
+    u64* slots;  // [4][workgroups]: three sets and the words of the roll call
     unsigned n;  // meetings so far
     int nwg;
 
@@ -47,6 +57,47 @@ struct Meeting {
             m = s > m ? s : m;
         }
         return m;
+    }
+
+    __host__ __device__ __forceinline__ u64* roll(int wg) const { return &slots[3 * (size_t)nwg + (size_t)wg]; }
+
+    // As a workgroup starts, after g launches; its value for the first meeting. ticks 0: nobody is present, whoever is
+    // on the device.
+    __host__ __device__ __forceinline__ u64 check_in(int wg, u64 g, u64 ticks) const {
+        const u64 was = M::swap(roll(wg), 2 * g, ticks ? 2 * g + 2 : 2 * g + 1);
+        return was == 2 * g && ticks ? SLOT_PRESENT : SLOT_REFUSED;
+    }
+    // The first meeting, after arrive() with the value of check_in: the verdict from every lanes-th word, SLOT_PRESENT,
+    // SLOT_REFUSED or, for a workgroup that checked in and stopped coming, SLOT_TIMEOUT.
+    __host__ __device__ __forceinline__ u64 call(int lane, int lanes, u64 g, u64 ticks, u64 most) const {
+        u64 m = SLOT_PRESENT;
+        for (int i = lane; i < nwg; i += lanes) {
+            u64 s = M::load(&set(n)[i]);
+            if (s == SLOT_EMPTY) {
+                const u64 t0 = M::now();
+                u64 limit = ticks;
+                do {
+                    M::pause();
+                    s = M::load(&set(n)[i]);
+                    if (s == SLOT_EMPTY && M::now() - t0 >= limit) {
+                        if (limit == most) s = SLOT_TIMEOUT;
+                        else if (M::swap(roll(i), 2 * g, 2 * g + 1) != 2 * g + 2) s = SLOT_REFUSED;
+                        limit = most;
+                    }
+                } while (s == SLOT_EMPTY);
+            }
+            m = s > m ? s : m;
+        }
+        return m;
+    }
+    // After a refused roll call: whether this workgroup is the last to leave.
+    __host__ __device__ __forceinline__ bool last_out(unsigned* left) const {
+        return M::add(left, 1u) == (unsigned)nwg - 1u;
+    }
+    // By the last to leave: the words as a launch that met leaves them.
+    __host__ __device__ __forceinline__ void clear_all(int lane, int lanes, u64 g) const {
+        for (int i = lane; i < 3 * nwg; i += lanes) M::store(&slots[i], SLOT_EMPTY);
+        for (int i = lane; i < nwg; i += lanes) M::store(roll(i), 2 * g + 2);
     }
 
     // Everybody has arrived, hence left the meeting before: its word is free again.

@@ -50,7 +50,9 @@ struct DEMParams {
     CylDev cyl[2];
     int spring;            // tangential spring with history (HYB_TANGENTIAL_SPRING) instead of the viscous law
     int allWalls;          // every wall within nebrRange is a contact partner (HYB_WALL_CONTACTS_ALL), not only the first
-    int* herr;             // the handle's error word (mapped pinned host memory), nullptr: none
+    int* herr;             // the handle's error word (mapped pinned host memory), nullptr: none; after it, the number
+                           // of steps done by one workgroup (dem_run.hip)
+    unsigned waitTicks;    // how long the workgroups of a step wait for each other at its start (10 ns)
 };
 
 // Wall-contact records per particle: one per wall with DEMParams::allWalls, else one.
@@ -142,7 +144,7 @@ struct DEMBuffers {
     double* pcor;          // [P][9]
     double* ppred;         // [P][9]
     double* pmn;           // [2 * pairCap][3]
-    // the whole-step kernel (dem_run.hip): barrier words [3][workgroups] (all ones: empty), which set comes next,
+    // the whole-step kernel (dem_run.hip): words of the workgroups [4][workgroups] (dem_barrier.h), which set comes next,
     // counts per workgroup [workgroups][RUN_COUNTS], exchange records [2][P][RUN_REC], pairs per particle [P],
     // unsorted per-particle pair lists and per element its pairs in order (and their springs) [2 * pairCap]
     unsigned long long* runSlots;
@@ -161,6 +163,9 @@ struct DEMBuffers {
 
 struct DEMRunState {
     unsigned barriers;
+    unsigned left;   // workgroups that have left a refused roll call
+    unsigned long long launches;
+    unsigned alone;  // steps done by one workgroup
 };
 struct DEMRunArgs {
     DEMParams p;

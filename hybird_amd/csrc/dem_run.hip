@@ -25,10 +25,12 @@
 //    the same barrier with device-scope release and acquire fences.
 //
 // Data that crosses workgroups between two fences (the exchange records, the barrier words) is read and written
-// with device-scope atomics only. All workgroups must be resident at once: dem_run_fits compares their number
-// with what the device holds, and larger beds use the per-launch kernels. Two such launches of one process cannot
-// wait for each other: all handles use one stream. A barrier that does not complete within
-// BARRIER_SECONDS (other processes holding the device) ends the launch with DEM_ERR_BARRIER.
+// with device-scope atomics only. All workgroups must be on the device at once: dem_run_fits compares their number
+// with what an otherwise idle device holds, and larger beds use the per-launch kernels. Two such launches of one
+// process cannot wait for each other, since all handles use one stream; where another process or a mask of the CUs
+// keeps some workgroups off the device, the roll call (dem_barrier.h) finds it out before anything is changed, and one
+// workgroup does the step. After the roll call a barrier that does not complete within BARRIER_SECONDS ends the launch
+// with DEM_ERR_BARRIER.
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -38,6 +40,7 @@
 #define HYB_DEM_POW_ATTR __attribute__((noinline))
 #include "dem_device.h"
 #include "dem_kernels.h"
+#include "dem_substep.h"
 #include "hybird_amd.h"
 
 namespace hyb {
@@ -47,6 +50,8 @@ namespace {
 constexpr u64 BITS_INF = 0x7FF0000000000000ull;
 constexpr u64 TICKS_PER_SECOND = 100000000;  // wall_clock64
 constexpr u64 BARRIER_SECONDS = 20;
+constexpr int ALONE_LANES = 256;
+constexpr int NOT_TOGETHER = -1;  // the roll call was refused
 constexpr int ENT_LANE = 8;  // neighbours per lane kept in LDS (4 x 8 per element; more are read from memory)
 constexpr uint32_t NO_GHOST = 0xFFFFFFFFu;
 
@@ -134,6 +139,13 @@ struct DeviceWords {
     static __device__ __forceinline__ void store(u64* w, u64 v) {
         __hip_atomic_store(w, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
+    static __device__ __forceinline__ u64 swap(u64* w, u64 from, u64 to) {
+        __hip_atomic_compare_exchange_strong(w, &from, to, __ATOMIC_RELAXED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        return from;
+    }
+    static __device__ __forceinline__ unsigned add(unsigned* w, unsigned v) {
+        return __hip_atomic_fetch_add(w, v, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
+    }
     static __device__ __forceinline__ u64 now() { return wall_clock64(); }
     static __device__ __forceinline__ void pause() { __builtin_amdgcn_s_sleep(1); }
 };
@@ -144,9 +156,10 @@ struct Grid : Meeting<DeviceWords> {
 
     // Maximum over the whole grid of `mine`; every store before it is visible to the exchange loads after it.
     // FULL: plain stores before it are visible to plain loads after it in every workgroup. Returns
-    // SLOT_TIMEOUT when the other workgroups did not arrive.
-    template <bool FULL>
-    __device__ __forceinline__ u64 meet(u64 mine) {
+    // SLOT_TIMEOUT when the other workgroups did not arrive. FIRST: the roll call after g launches, waiting `ticks` for
+    // each workgroup; the verdict.
+    template <bool FULL, bool FIRST = false>
+    __device__ __forceinline__ u64 meet(u64 mine, u64 g = 0, u64 ticks = 0) {
         constexpr int W = ONE ? 8 : 4;  // wavefronts
         __shared__ u64 red[2][W], all[W];
         const int wave = (int)(threadIdx.x >> 6);
@@ -169,7 +182,11 @@ struct Grid : Meeting<DeviceWords> {
                 if constexpr (FULL) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
                 arrive((int)blockIdx.x, v);
             }
-            const u64 m = wave_max_last(wait_all((int)threadIdx.x, (int)blockDim.x, BARRIER_SECONDS * TICKS_PER_SECOND));
+            constexpr u64 MOST = BARRIER_SECONDS * TICKS_PER_SECOND;
+            u64 m;
+            if constexpr (FIRST) m = call((int)threadIdx.x, (int)blockDim.x, g, ticks, MOST);
+            else m = wait_all((int)threadIdx.x, (int)blockDim.x, MOST);
+            m = wave_max_last(m);
             if ((threadIdx.x & 63) == 63) all[wave] = m;
             __syncthreads();
 #pragma unroll
@@ -784,6 +801,61 @@ __device__ __forceinline__ void touch(const DEMParams& p, const DEMBuffers& b, c
     }
 }
 
+// ------------------------------------------------------------------ a step by one workgroup
+// After a refused roll call: the whole step by the last workgroup to leave, on the state in memory, with the sub-steps
+// of dem_substep.h (the same operations: the same results). Slow (ten sub-steps, one with a rebuild, 2.7 ms at 1,000
+// spheres and 40 at 20,000, against 0.06 and 0.7 by all), so the host, told by the word after the handle's error word,
+// then takes the launches of dem.hip for a while.
+__device__ __forceinline__ void alone_sync() {
+    __threadfence();  // also what the atomics of the part before left in memory
+    __syncthreads();
+}
+template <bool SP, bool CL>
+__device__ __attribute__((noinline)) void not_together(const DEMRunArgs* a, int nsub, int force) {
+    __shared__ int last;
+    const DEMParams& p = a->p;
+    const DEMBuffers& b = a->b;
+    const int t = (int)threadIdx.x, lanes = (int)blockDim.x;
+    const Meeting<DeviceWords> m{b.runSlots, 0u, (int)gridDim.x};
+    const u64 g = b.st2->launches;
+    if (t == 0) last = m.last_out(&b.st2->left) ? 1 : 0;
+    __syncthreads();
+    if (!last) return;
+    const El E{b.el, p.E};
+    for (int sub = 0; sub < (force ? 1 : nsub); ++sub) {
+        alone_sync();
+        rebuild_by_one<ALONE_LANES>(p, b, force);
+        if (force) break;
+        alone_sync();
+        if (b.st->error) return;
+        const int T = b.st->nPairs;
+        for (int k = t; k < T; k += lanes) eval_pair<SP, CL>(p, b, E, k);
+        alone_sync();
+        u64 vm = 0;
+        for (int e = t; e < p.E; e += lanes) {
+            const double v2 = gather_elem<SP, CL>(p, b, e);
+            const u64 bits = v2 <= 1.79769313486231570e308 ? (u64)__double_as_longlong(v2) : BITS_INF;
+            vm = bits > vm ? bits : vm;
+        }
+        vm = wave_max_last(vm);
+        if ((t & 63) == 63) atomicMax(reinterpret_cast<u64*>(b.vmax), vm);
+    }
+    alone_sync();
+    if (b.st->error) return;
+    for (int q = t >> 2; q < p.E; q += lanes >> 2) {
+        const int ilo = CL ? b.efirst[q] : q;
+        element_entries(p, b, ilo, CL ? b.efirst[q + 1] - ilo : 1, t & 3);
+    }
+    m.clear_all(t, lanes, g);
+    __syncthreads();
+    if (t == 0) {
+        b.st2->left = 0;
+        b.st2->launches += 1;
+        if (!force) b.st2->alone += 1;
+        if (p.herr) __hip_atomic_store(p.herr + 1, (int)b.st2->alone, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+}
+
 // ------------------------------------------------------------------ the kernel
 // ONE: the grid is one workgroup (up to 512 lanes, 128 elements; with multi-sphere elements 256 and 64);
 // otherwise 256 lanes, 64 elements each.
@@ -800,6 +872,8 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
     const int size = e0 < p.E ? (CL ? b.efirst[e + 1] - ilo : 1) : 0;
     const bool multi = CL && size > 1;
     Grid<ONE> grid{{b.runSlots, b.st2->barriers, (int)gridDim.x}, (int)(blockDim.x >> 6)};
+    u64 checked = SLOT_PRESENT;
+    if (!ONE && threadIdx.x == 0) checked = grid.check_in((int)blockIdx.x, b.st2->launches, b.runArgs->p.waitTicks);
     u64 vm = *reinterpret_cast<const u64*>(b.vmax);
     double maxDisp = b.st->maxDisp;
     V3 proto;
@@ -885,7 +959,11 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
             __threadfence_block();
         }
         publish<CL, ONE>(recs.base, ilo, size, c, S, proto);
-        if (grid.template meet<false>(0) == SLOT_TIMEOUT) err = DEM_ERR_BARRIER;
+        if constexpr (ONE) (void)grid.template meet<false>(0);
+    }
+    if constexpr (!ONE) {  // up to here nothing that outlives the launch has been changed
+        const u64 verdict = grid.template meet<false, true>(checked, b.st2->launches, b.runArgs->p.waitTicks);
+        if (verdict != SLOT_PRESENT) err = verdict == SLOT_REFUSED ? NOT_TOGETHER : DEM_ERR_BARRIER;
     }
     V3 FP, MP, FW, MW;
     int done = 0;
@@ -1126,6 +1204,12 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
         done = sub + 1;
         if (vm == SLOT_TIMEOUT) err = DEM_ERR_BARRIER;
     }
+    if constexpr (!ONE) {
+        if (err == NOT_TOGETHER) {
+            not_together<SP, CL>(b.runArgs, nsub, force);
+            return;
+        }
+    }
     // ---- state of the last completed sub-step
     if (done && size) {
         double xp[6], qp[6], wp[6];
@@ -1195,6 +1279,7 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
                 *reinterpret_cast<u64*>(b.vmax) = vm;
                 b.st->maxDisp = maxDisp;
             }
+            if (!ONE) b.st2->launches += 1;
             b.st2->barriers = grid.n % 3u + 3u;  // only the set that comes next and the parity of the LDS words matter
         }
     }

@@ -365,6 +365,8 @@ void DEM::discreteElementGet(GetPot& lbmCfgFile, GetPot& command_line) {  // DEM
         ASSERT(wc == "FIRST" || wc == "ALL");
         cfg_.wallContacts = wc == "ALL" ? HYB_WALL_CONTACTS_ALL : HYB_WALL_CONTACTS_FIRST;
     }
+    // extension: how long the workgroups of a step wait for each other (nanoseconds; 0: the default, negative: never)
+    cfg_.demStepWait = extension_key<int>(lbmCfgFile, command_line, "demStepWait", 0);
     // particle initial state (DEM.cpp:63-116)
     string particleFile;
     PARSE_CLASS_MEMBER(lbmCfgFile, particleFile, "particleFile", "particles.dat");

@@ -31,6 +31,7 @@ DEM_FIELDS = {"walls": (np.float64, (-1, 12)), "objectForces": (np.float64, (-1,
               "p_data": (np.float64, (-1, 10)), "p_idx": (np.uint32, (-1, 4)), "neighborTable": (np.uint32, None),
               "nearWallTable": (np.uint32, None), "ghostIndex": (np.uint32, None), "ghostVec": (np.float64, (-1, 3)),
               "dem_scalars": (np.float64, None), "rebuilds": (np.float64, None), "energy": (np.float64, None),
+              "alone_steps": (np.float64, None),
               "nearObjectTable": (np.uint32, None), "objects": (np.float64, (-1, 8))}
 
 # every extern "C" entry point declared in include/hybird_amd.h

@@ -133,7 +133,15 @@ typedef struct hyb_config {
     double frictionCoefFluid; /* HYB_RHEOLOGY_FRICTIONAL: yield stress per unit gauge pressure */
     int32_t tangentialModel;  /* HYB_TANGENTIAL_VISCOUS (reference) or HYB_TANGENTIAL_SPRING */
     int32_t wallContacts;     /* HYB_WALL_CONTACTS_FIRST (reference) or HYB_WALL_CONTACTS_ALL */
-    int32_t reserved[2];
+    /* Beds of more than 128 elements (64 with multi-sphere elements) step in one launch whose workgroups wait for each
+     * other, up to about 32,000 elements on a device of 256 CUs. demStepWait: nanoseconds they wait at the start of a
+     * step until all are on the device (0: 20 ms). If another process, or a mask of its CUs, keeps some of them off
+     * for longer, one workgroup does the step alone, with the same results, and the handle's next 256 steps (twice as
+     * many each further time) take three launches per sub-step instead; the view "alone_steps" counts such steps.
+     * Negative: always three launches per sub-step, for a device that is known to be shared. Below 10: always one
+     * workgroup. */
+    int32_t demStepWait;
+    int32_t reserved[1];
 } hyb_config;
 
 /* Fills *cfg with the reference's parse defaults (LB.cpp:93-185, DEM.cpp:15-181)
@@ -198,7 +206,8 @@ int hyb_cycle(hyb_lb* lb, hyb_dem* dem, int32_t n);
  *       "p_data" f64[P][10] (x0, x1, radiusVec, r), "p_idx" u32[P][4],
  *       "neighborTable" u32[2*pairs], "nearWallTable" u32[2*k], "ghostIndex" u32[G], "ghostVec" f64[G][3],
  *       "nearObjectTable" u32[2*k] (particle, object), "objects" f64[O][8] (index, r, x0, x1),
- *       "dem_scalars" f64[17], "energy" f64[6] (DEM::particleEnergy after the last sub-step: kin, rotKin,
+ *       "dem_scalars" f64[17], "rebuilds" f64[1] (neighbour rebuilds), "alone_steps" f64[1] (see demStepWait),
+ *       "energy" f64[6] (DEM::particleEnergy after the last sub-step: kin, rotKin,
  *       trKin, grav, elastic, total; DEM.cpp:2226-2276), "walls" f64[W][12] (p, n, FParticle, FHydro = 0:
  *       walls[] after the last sub-step, DEM.cpp:1936-1979), "objectForces" f64[O][3] (objects[].FParticle,
  *       DEM.cpp:2100-2134; rows as "objects")

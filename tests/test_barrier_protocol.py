@@ -35,6 +35,7 @@ struct HostWords {  // 1 tick: 1 us
         __atomic_compare_exchange_n(w, &from, to, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST);
         return from;
     }
+    static unsigned add(unsigned* w, unsigned v) { return __atomic_fetch_add(w, v, __ATOMIC_SEQ_CST); }
     static u64 now() {
         return (u64)std::chrono::duration_cast<std::chrono::microseconds>(
             std::chrono::steady_clock::now().time_since_epoch()).count();
@@ -72,7 +73,7 @@ def test_every_meeting_gives_every_workgroup_the_maximum(tmp_path):
     _run(tmp_path, r"""
 int main() {
     for (int nwg : {2, 3, 7}) {
-        std::vector<u64> words(3 * nwg, SLOT_EMPTY);
+        std::vector<u64> words(4 * nwg, SLOT_EMPTY);
         unsigned kept = 0;
         for (int l = 0; l < 40; ++l) {
             const int meetings = 1 + l % 5;
@@ -103,7 +104,7 @@ def test_a_wait_that_ends_without_the_others_is_reported(tmp_path):
     _run(tmp_path, r"""
 int main() {
     const int nwg = 3;
-    std::vector<u64> words(3 * nwg, SLOT_EMPTY);
+    std::vector<u64> words(4 * nwg, SLOT_EMPTY);
     std::atomic<int> error{0}, gone{0};
     launch(nwg, [&](int wg) {
         Meeting<HostWords> m{words.data(), 0, nwg};
@@ -116,6 +117,65 @@ int main() {
         if (leaving(wg, v == SLOT_TIMEOUT ? 7 : 0) == LEAVE_ERROR) error = 7;
     });
     check(error == 7, "the launch is reported as failed");
+    return 0;
+}
+""")
+
+
+def test_a_roll_call_has_one_verdict(tmp_path):
+    """Workgroups that are late at random, against a short wait: all come to the same verdict; a refused launch is done
+    once, by the last to leave; the launches after it meet as ever."""
+    _run(tmp_path, r"""
+int main() {
+    int together = 0, apart = 0;
+    for (int nwg : {2, 5}) {
+        std::vector<u64> words(4 * nwg, SLOT_EMPTY);
+        for (int wg = 0; wg < nwg; ++wg) words[3 * nwg + wg] = 0;
+        unsigned kept = 0, left = 0;
+        for (int l = 0; l < 150; ++l) {
+            const unsigned from = kept;
+            std::atomic<int> present{0}, refused{0}, done{0};
+            const u64 wait = l % 10 == 0 ? 0 : 1500;
+            launch(nwg, [&](int wg) {
+                std::mt19937 rng(1000 * l + wg);
+                if (rng() % 4 == 0) late((int)(rng() % 4));
+                Meeting<HostWords> m{words.data(), from, nwg};
+                const u64 checked = m.check_in(wg, l, wait);
+                if (rng() % 4 == 0) late((int)(rng() % 3));
+                m.arrive(wg, checked);
+                const u64 verdict = m.call(0, 1, l, wait, LONG);
+                if (verdict == SLOT_REFUSED) {
+                    ++refused;
+                    if (m.last_out(&left)) {
+                        check(refused == nwg, "everybody has left");
+                        m.clear_all(0, 1, l);
+                        left = 0;
+                        ++done;
+                    }
+                    return;
+                }
+                check(verdict == SLOT_PRESENT, "present or refused");
+                m.free_last(wg);
+                ++m.n;
+                ++present;
+                for (int k = 0; k < 1 + l % 4; ++k) {
+                    m.arrive(wg, (u64)(10 * k + wg));
+                    check(m.wait_all(0, 1, LONG) == (u64)(10 * k + nwg - 1), "maximum after the roll call");
+                    m.free_last(wg);
+                    ++m.n;
+                }
+                if (leaving(wg, 0) == LEAVE_STATE) {
+                    kept = m.n % 3u + 3u;
+                    ++done;
+                }
+            });
+            check((present == nwg && refused == 0) || (present == 0 && refused == nwg), "one verdict");
+            check(done == 1, "the step is done once");
+            check(wait || refused == nwg, "no wait, nobody present");
+            (refused ? apart : together) += 1;
+        }
+    }
+    check(together > 10 && apart > 10, "both verdicts occur");
     return 0;
 }
 """)
