@@ -987,6 +987,20 @@ int hyb_dem_set_save_count(hyb_dem* d, int32_t saveCount) {
     return HYB_OK;
 }
 
+// Whether a step of `multiStep` sub-steps is faster in one launch (launch_dem_run) than in three per sub-step. The
+// launch loads and stores every element's state, lists and springs once, which takes as long as one sub-step's three
+// launches, or with springs two. us a step, one launch / three per sub-step, beds at 0.17 by volume with one rebuild in
+// 1,000 sub-steps: one sub-step 30 spheres 15.0 / 16.0, 64 19.1 / 17.6, 128 27.5 / 18.3, 1,000 25.0 / 19.9, 7,728
+// 28.5 / 24.6, 30,000 44.8 / 47.0; with springs 30 19.2 / 16.3, 1,000 34.4 / 20.6, 20,000 54.7 / 39.7; two sub-steps 128
+// 35.5 / 36.3, 1,000 33.3 / 40.3; with springs 30 24.4 / 33.0, 1,000 44.5 / 40.9, 7,728 49.2 / 51.9, three 1,000 54.6 /
+// 61.8. 65 clumps 24.2 / 27.7, with springs 29.3 / 28.5, 5,000 30.0 / 40.0 and 36.6 / 41.1. Above 4,096 spheres without
+// springs one launch stays, for its rebuild: 20,000 spheres 43.2 / 36.7, but a rebuild 0.5 / 5 ms.
+static bool one_launch_pays(const hyb_dem* d) {
+    const DEMParams& p = d->p;
+    const int least = p.clumps ? 1 : 1 + (p.E > 64 && p.E <= 4096 ? 1 : 0) + (p.spring ? 1 : 0);
+    return d->multiStep >= least;
+}
+
 int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
     if (!d || !d->inited) return fail(HYB_E_STATE, "hyb_dem_step before hyb_dem_init");
     if (int rc = dem_pending(d)) return rc;
@@ -997,7 +1011,7 @@ int hyb_dem_step(hyb_dem* d) {  // DEM.cpp:331-376
         d->apart = d->apartNext;
         d->apartNext = std::min(2 * d->apartNext, STEPS_APART_MOST);
     }
-    const bool whole = d->wholeStep && !d->saveCount && !d->apart;
+    const bool whole = d->wholeStep && !d->saveCount && !d->apart && one_launch_pays(d);
     if (d->apart) --d->apart;
     for (int it = 0; it < d->multiStep; ++it) {
         d->demTimeStep++;
