@@ -93,33 +93,29 @@ __device__ __forceinline__ T link_in(int j, uint8_t tl, T fsj, T vn, double mL, 
     if (tl == T_WALL_MOVING) a = 1.0 * nd.mi;  // zero velocity, so half-way bounce-back as at a static wall
     return fsj;
 }
-// Any link, in the pull form or before the first collision (f = fs).
+// The other links (slip walls, cylinders), and any link before the first collision (f = fs).
 template <typename T, bool SHIFT>
-__device__ __forceinline__ T any_link(int j, bool pull, uint8_t tl, T fsj, const T* __restrict__ fpost,
-                                      const uint8_t* __restrict__ type, const double* __restrict__ mass, const MassNode& nd,
-                                      const LBKParams& p, double& a) {
+__device__ __forceinline__ T wall_in(int j, bool pull, uint8_t tl, T fsj, const T* __restrict__ fpost,
+                                     const uint8_t* __restrict__ type, const double* __restrict__ mass, const MassNode& nd,
+                                     const LBKParams& p, double& a) {
 #pragma clang fp contract(off)
     const double mi = nd.mi;
     const auto active = [&](size_t n) { const uint8_t t = type[n]; return t == T_FLUID || t == T_INTERFACE; };
     // moving walls have zero velocity. Mass exchange: a = m for a moving wall, the slip rule for a moving slip wall
     // (LB.cpp:1531-1575), else 0.
-    const auto slip_share = [&]() {
+    a = 0.0;
+    if (tl == T_WALL_MOVING || tl == T_CURVED) {  // LB.cpp:1539-1545
+        a = 1.0 * mi;
+    } else if (tl == T_SLIP_MOVING) {
         bool half = false;
         if (j > 6) {
             const bool a1 = active(nb_index(p, nd.c, slip1check(j))), a2 = active(nb_index(p, nd.c, slip2check(j)));
             half = (a1 && !a2) || (!a1 && a2);
         }
-        return half ? 0.0 + 1.0 * p.slipS2 * mi : 0.0 + 1.0 * mi;
-    };
-    const size_t L = nb_index(p, nd.c, j);
-    if (pull && plain_link(tl))
-        return link_in<T, SHIFT>(j, tl, fsj, fpost[(size_t)opp(j) * p.PS + L], mass[L], nd, p.initDensity, a);
-    a = 0.0;
-    if (tl == T_WALL_MOVING) a = 1.0 * mi;
-    else if (tl == T_SLIP_MOVING) a = slip_share();
-    else if (tl == T_CURVED) a = 1.0 * mi;  // LB.cpp:1539-1545
+        a = half ? 0.0 + 1.0 * p.slipS2 * mi : 0.0 + 1.0 * mi;
+    }
     if (!pull) {
-        if (tl == T_INTERFACE) a = 0.5 * (mass[L] + mi);
+        if (tl == T_INTERFACE) a = 0.5 * (mass[nb_index(p, nd.c, j)] + mi);
         else if (tl == T_FLUID) a = 1.0;
         return fpost[(size_t)opp(j) * p.PS + nd.idx];
     }
@@ -131,8 +127,12 @@ __device__ __forceinline__ T any_link(int j, bool pull, uint8_t tl, T fsj, const
 
 // Bound by memory latency and by the lines it touches: about 400 bytes a node where neighbouring lanes hold
 // neighbouring nodes (FP32: 262,144 nodes of one z plane 147 us with the list as the atomics left it and one
-// wavefront per SIMD, 33 now). PLAIN: after a collision, in a lattice without slip walls and cylinders; otherwise links are
-// taken one at a time (unrolled as well, those rules left one wavefront per SIMD).
+// wavefront per SIMD, 33 now). PLAIN: after a collision, in a lattice without slip walls and cylinders. Otherwise the
+// links to those are taken one at a time before the plain ones, whose loads still go together; their exchange waits in
+// LDS, so that a node's exchange is added in the order of its links. us, all links one at a time / with every rule in
+// the unrolled loop / so: slip walls, 256 x 128 x 128 nodes FP64 52.7 / 45.5 / 35.0, FP32 51.6 / 44.4 / 34.8, 101 x 47 x 66
+// FP64 40.7 / 39.9 / 26.3, a cylinder in 56 x 40 x 40 49.2 / 43.0 / 30.6. Bounded to three wavefronts per SIMD, as the
+// plain form is, it spills (49.4 and 42.6).
 template <typename T, bool SHIFT, bool PLAIN>
 __global__ void __launch_bounds__(MASS_BLOCK, PLAIN ? (sizeof(T) == 4 ? 4 : 3) : 1)
     k_fs_mass(const T* __restrict__ fpost, T* __restrict__ fout, const uint8_t* __restrict__ type,
@@ -140,6 +140,7 @@ __global__ void __launch_bounds__(MASS_BLOCK, PLAIN ? (sizeof(T) == 4 ? 4 : 3) :
               const uint32_t* __restrict__ list, FSCounters* __restrict__ ctr, int cur, double* __restrict__ mnew,
               uint8_t* __restrict__ state, LBKParams p, int pull) {
 #pragma clang fp contract(off)
+    __shared__ double otherDm[PLAIN ? 1 : 18][MASS_BLOCK];
     const size_t N = (size_t)p.X * p.Y * p.Z;
     const uint32_t nI = ctr->n[cur];
     if (blockIdx.x == 0 && threadIdx.x == 0) {  // counters of this step's later phases
@@ -170,41 +171,47 @@ __global__ void __launch_bounds__(MASS_BLOCK, PLAIN ? (sizeof(T) == 4 ? 4 : 3) :
         nd.mi = mass[idx];
         nd.u = V3(uS[idx], uS[N + idx], uS[2 * N + idx]);
         nd.usq = nd.u.norm2();
-        double dm = 0.0;
-        if constexpr (PLAIN) {
-            // every neighbour's type and mass and its opposite population, loaded together before any is used (a
-            // neighbour index is always a node of the lattice, so the loads a neighbour's type makes unnecessary
-            // stay in bounds): one round trip instead of one per link
-            T fs[19], vn[19];
-            uint8_t tn[19];
-            double mL[19];
+        // every neighbour's type and mass and its opposite population, loaded together before any is used (a
+        // neighbour index is always a node of the lattice, so the loads a neighbour's type makes unnecessary
+        // stay in bounds): one round trip instead of one per link
+        T fs[19], vn[19];
+        uint8_t tn[19];
+        double mL[19];
 #pragma unroll
-            for (int j = 0; j < 19; ++j) fs[j] = fpost[(size_t)j * p.PS + idx];
+        for (int j = 0; j < 19; ++j) fs[j] = fpost[(size_t)j * p.PS + idx];
 #pragma unroll
-            for (int j = 1; j < 19; ++j) {
-                const uint32_t L = nb(j);
-                tn[j] = type[L];
-                vn[j] = fpost[(size_t)opp(j) * p.PS + L];
-                mL[j] = mass[L];
-            }
-            fout[idx] = fs[0];
+        for (int j = 1; j < 19; ++j) {
+            const uint32_t L = nb(j);
+            tn[j] = type[L];
+            vn[j] = fpost[(size_t)opp(j) * p.PS + L];
+            mL[j] = mass[L];
+        }
+        fout[idx] = fs[0];
+        uint32_t other = 0;  // links that are not plain
+        if constexpr (!PLAIN) {
 #pragma unroll
-            for (int j = 1; j < 19; ++j) {
-                double a;
-                const T v = link_in<T, SHIFT>(j, tn[j], fs[j], vn[j], mL[j], nd, p.initDensity, a);
-                fout[(size_t)opp(j) * p.PS + idx] = v;
-                dm += 1.0 * a * (to_d(v) - to_d(fs[j]));
-            }
-        } else {
-            fout[idx] = fpost[idx];
-#pragma unroll 1
-            for (int j = 1; j < 19; ++j) {
+            for (int j = 1; j < 19; ++j)
+                if (!pull || !plain_link(tn[j])) other |= 1u << j;
+            for (uint32_t rest = other; rest; rest &= rest - 1u) {
+                const int j = __ffs((int)rest) - 1;
                 double a;
                 const T fsj = fpost[(size_t)j * p.PS + idx];
-                const T v = any_link<T, SHIFT>(j, pull != 0, type[nb_index(p, nd.c, j)], fsj, fpost, type, mass, nd, p, a);
+                const T v = wall_in<T, SHIFT>(j, pull != 0, type[nb_index(p, nd.c, j)], fsj, fpost, type, mass, nd, p, a);
                 fout[(size_t)opp(j) * p.PS + idx] = v;
-                dm += 1.0 * a * (to_d(v) - to_d(fsj));
+                otherDm[j - 1][threadIdx.x] = 1.0 * a * (to_d(v) - to_d(fsj));
             }
+        }
+        double dm = 0.0;
+#pragma unroll
+        for (int j = 1; j < 19; ++j) {
+            if (!PLAIN && (other >> j & 1u)) {
+                dm += otherDm[PLAIN ? 0 : j - 1][threadIdx.x];
+                continue;
+            }
+            double a;
+            const T v = link_in<T, SHIFT>(j, tn[j], fs[j], vn[j], mL[j], nd, p.initDensity, a);
+            fout[(size_t)opp(j) * p.PS + idx] = v;
+            dm += 1.0 * a * (to_d(v) - to_d(fs[j]));
         }
         const double mn = nd.mi + dm;
         const double n = to_d(rho[idx]);
