@@ -148,12 +148,14 @@ struct Arena {
     std::vector<void*> slabs;
     char* next = nullptr;
     size_t left = 0, slab = (size_t)4 << 20;
+    size_t expected = 0;  // bytes still to come, where the owner says so: the last slab is no larger
+    static size_t rounded(size_t bytes) { return (bytes + ARENA_ALIGN - 1) / ARENA_ALIGN * ARENA_ALIGN; }
     int take(void** p, size_t bytes) {
         *p = nullptr;
         if (bytes == 0) return HYB_OK;
-        bytes = (bytes + ARENA_ALIGN - 1) / ARENA_ALIGN * ARENA_ALIGN;
+        bytes = rounded(bytes);
         if (bytes > left) {
-            const size_t size = std::max(bytes, slab);
+            const size_t size = std::max(bytes, expected ? std::min(slab, expected) : slab);
             void* q = nullptr;
             const hipError_t e = hipMalloc(&q, size);
             if (e != hipSuccess) {
@@ -161,12 +163,15 @@ struct Arena {
                 return fail(HYB_E_HIP, std::string("device allocation: ") + hipGetErrorString(e));
             }
             slabs.push_back(q);
+            expected -= std::min(expected, bytes);
             if (size > slab) {  // the rest of the current slab stays in use
                 *p = q;
                 return HYB_OK;
             }
             next = (char*)q;
             left = size;
+        } else {
+            expected -= std::min(expected, bytes);
         }
         *p = next;
         next += bytes;
@@ -177,7 +182,7 @@ struct Arena {
         for (void* q : slabs) (void)hipFree(q);
         slabs.clear();
         next = nullptr;
-        left = 0;
+        left = expected = 0;
     }
 };
 
@@ -1558,9 +1563,9 @@ int hyb_adj_forward(hyb_lb* l, hyb_dem* d, int32_t steps, int32_t every) {
     // ms), a state of 128^3 nodes has one of its own. Larger slabs for these made the first gradient of a process
     // slower (199 ms; slabs of 1 GiB 216, one of 10 GB 360 to 1400, one per state 186) and a repeated one only 5 %
     // faster.
-    const size_t need = 8 * adj_tau_slots(l->params()) + 24 * l->N + pb * (size_t)(M + K + 2) + ARENA_ALIGN * (size_t)(M + K + 4);
-    const size_t one = (pb + ARENA_ALIGN - 1) / ARENA_ALIGN * ARENA_ALIGN;
-    l->adjArena.slab = std::min(need, one * std::max<size_t>(1, ((size_t)256 << 20) / one));
+    const size_t one = Arena::rounded(pb);
+    l->adjArena.slab = one * std::max<size_t>(1, ((size_t)256 << 20) / one);
+    l->adjArena.expected = one * (size_t)(M + K + 2) + Arena::rounded(24 * l->N) + Arena::rounded(8 * adj_tau_slots(l->params()));
     const auto grab = [&](std::vector<void*>& v, int n) -> int {
         for (int m = 0; m < n; ++m) {
             void* q = nullptr;
