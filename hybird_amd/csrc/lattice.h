@@ -65,14 +65,17 @@ __device__ __forceinline__ bool row_coord(const LBKParams& p, Coord& c) {
 // alone lost (X = 150: 34.9 and 42.0, FP64 67.7 and 73.0). 64 consecutive nodes of the whole lattice per wavefront
 // (32.8, FP64 58.8) would cut the run sums below elsewhere and change their rounding.
 constexpr int MERGE_RUN = 16, XCDS = 8;
-inline bool merge_map(const LBKParams& p, Prec prec) {
-    return (size_t)p.X * (prec == Prec::F64 ? 8 : 4) % 128 != 0;
-}
-inline dim3 merge_grid(const LBKParams& p) {
+inline size_t merge_blocks(const LBKParams& p) {
     const dim3 g = row_grid(p);
     const size_t n = (size_t)g.x * g.y * g.z, per = (size_t)MERGE_RUN * XCDS;
-    return dim3((unsigned)((n + per - 1) / per * per), 1, 1);
+    return (n + per - 1) / per * per;
 }
+// A launch holds less than 2^32 lanes along x: a lattice a few nodes wide in x can have more lanes than that (X = 3 from
+// 8,192 x 8,192 on).
+inline bool merge_map(const LBKParams& p, Prec prec) {
+    return (size_t)p.X * (prec == Prec::F64 ? 8 : 4) % 128 != 0 && merge_blocks(p) * row_block(p).x < ((size_t)1 << 32);
+}
+inline dim3 merge_grid(const LBKParams& p) { return dim3((unsigned)merge_blocks(p), 1, 1); }
 // n / d for inv = ceil(2^64 / d), 0 for d = 1: the error n (inv d - 2^64) / (d 2^64) is below 1 / d for 32-bit n, d.
 inline uint64_t inverse_of(uint64_t d) { return d == 1 ? 0ull : ~0ull / d + 1ull; }
 __device__ __forceinline__ uint32_t div_by(uint32_t n, uint64_t inv) {
