@@ -199,7 +199,7 @@ __device__ __forceinline__ void rebuild_by_one(const DEMParams& p, const DEMBuff
     __syncthreads();
     for (int s = t; s < S; s += RB) {
         const int c = linearize(slot_pos(E, p, b, s), p.cellWidth, p.nCells) + S;
-        if (c < 0 || c >= S + nc) {
+        if (c < S || c >= S + nc) {  // below S: a slot, not a cell
             sh_err = 2;
             b.cellOf[s] = 0;
         } else {
