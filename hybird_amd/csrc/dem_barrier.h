@@ -7,11 +7,11 @@
 //
 // A launch begins with a roll call, since nothing promises that its workgroups are on the device together: another
 // process's work, or a mask, may leave too few CUs, and two such launches of two processes can each hold a part and
-// wait for the other. Each workgroup has one more word, 2 g after g launches, and checks in as it starts: 2 g + 2. At
-// the first meeting, a workgroup that has waited long enough for another refuses it, by making that word 2 g + 1,
-// unless the other has checked in and is only on its way. A word changes once, so the launch meets if all have checked
-// in, and otherwise nobody sees everybody arrive: one that was refused says so when it comes. Then all leave, and the
-// last to leave does the work alone. Checking in so early takes it out of the way of the first meeting.
+// wait for the other. Each workgroup has one more word, 2 g after g launches, and checks in before the first meeting:
+// 2 g + 2. At that meeting, a workgroup that has waited long enough for another refuses it, by making that word
+// 2 g + 1, unless the other has checked in and is only on its way. A word changes once, so the launch meets if all have
+// checked in, and otherwise nobody sees everybody arrive: one that was refused says so when it comes. Then all leave,
+// and the last to leave does the work alone.
 //
 // M: the memory of the words, with load, store, swap (compare and swap; the old value), add (the old value), now (in
 // ticks) and pause.
@@ -61,7 +61,7 @@ struct Meeting {
 
     __host__ __device__ __forceinline__ u64* roll(int wg) const { return &slots[3 * (size_t)nwg + (size_t)wg]; }
 
-    // As a workgroup starts, after g launches; its value for the first meeting. ticks 0: nobody is present, whoever is
+    // Before the first meeting, after g launches; the value to arrive with there. ticks 0: nobody is present, whoever is
     // on the device.
     __host__ __device__ __forceinline__ u64 check_in(int wg, u64 g, u64 ticks) const {
         const u64 was = M::swap(roll(wg), 2 * g, ticks ? 2 * g + 2 : 2 * g + 1);

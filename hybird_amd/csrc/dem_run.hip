@@ -5,10 +5,12 @@
 // memory latency and one lane's serial Gear update. Here the element state stays on chip over all sub-steps of
 // the call, four lanes per element, and workgroups exchange only the predicted position, velocity and angular
 // velocity (96 bytes per particle, two buffers) and one word each for the displacement maximum. What bounds a
-// sub-step now is the serial FP64 chain of one wavefront (about 13,000 cycles with a touching pair: pow, square
-// roots, divisions) and, with several workgroups, two trips to memory (the barrier's words, the partners' records).
-// DEM step of ten sub-steps, before -> now: 6 spheres 140 -> 60 us, 100 spheres 171 -> 60, 561 (spring) 190 -> 110,
-// 7,728 220 -> 115, 20,000 (two per SIMD) 330 -> 165; 600 clumps 440 -> 120.
+// sub-step now is latency: in one workgroup (100 spheres) a wavefront lives about 15,000 cycles per sub-step, issues
+// VALU instructions (the FP64 chain, with pow, square roots and divisions in a touching pair) in 26 % of them and
+// waits at a counter or a barrier in 47 %. Over several workgroups, with two trips to memory per sub-step (the barrier's
+// words, the partners' records), it lives 29,000 to 39,000 cycles, issues in 15 to 23 % and waits in 60 to 65 %.
+// DEM step of ten sub-steps, before -> now, us: 6 spheres 140 -> 60, 100 spheres 171 -> 62, 561 (spring) 190 -> 131,
+// 7,728 220 -> 122, 20,000 (two workgroups per CU) 330 -> 167; 600 clumps 440 -> 117.
 //
 //  * Lane c of an element's quad holds component c of position, angular velocity and orientation (lane 3: only
 //    the quaternion's last component and the particle's radius and mass), so the Gear predictor and corrector
@@ -243,8 +245,8 @@ __device__ __forceinline__ void wg_offsets(const int* cnt, int nwg, int col, int
 }
 
 // Exclusive scan of a[0..n) over the grid, each workgroup on its own contiguous part; results to o1 and o2
-// (may be a). Two columns of the per-workgroup counts are used in turn. Returns a barrier error or 0; readers
-// of the result need a further barrier.
+// (may be a). col: a column of the per-workgroup counts, free again after the next barrier. Returns a barrier error or
+// 0; readers of the result need a further barrier.
 template <bool ONE>
 __device__ __forceinline__ int grid_exscan(Grid<ONE>& grid, const DEMBuffers& b, const int* a, int n, int* o1, int* o2, int col, int& total) {
     const int len = (n + grid.nwg - 1) / grid.nwg;
@@ -872,8 +874,6 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
     const int size = e0 < p.E ? (CL ? b.efirst[e + 1] - ilo : 1) : 0;
     const bool multi = CL && size > 1;
     Grid<ONE> grid{{b.runSlots, b.st2->barriers, (int)gridDim.x}, (int)(blockDim.x >> 6)};
-    u64 checked = SLOT_PRESENT;
-    if (!ONE && threadIdx.x == 0) checked = grid.check_in((int)blockIdx.x, b.st2->launches, b.runArgs->p.waitTicks);
     u64 vm = *reinterpret_cast<const u64*>(b.vmax);
     double maxDisp = b.st->maxDisp;
     V3 proto;
@@ -948,6 +948,11 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
         }
     };
     int err = 0, buf = 0;
+    u64 checked = SLOT_PRESENT;
+    const auto check_in = [&]() {
+        if (!ONE && threadIdx.x == 0) checked = grid.check_in((int)blockIdx.x, b.st2->launches, b.runArgs->p.waitTicks);
+    };
+    if (force) check_in();
     if (!force) {
         load_lists();
         if constexpr (SP) {
@@ -958,6 +963,7 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
                 }
             __threadfence_block();
         }
+        check_in();  // before the stores, whose completion is waited for anyway; loads after it would wait for it
         publish<CL, ONE>(recs.base, ilo, size, c, S, proto);
         if constexpr (ONE) (void)grid.template meet<false>(0);
     }
