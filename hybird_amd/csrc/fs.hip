@@ -42,9 +42,9 @@ constexpr int FS_GRID = 1024;
 // k_fs_mass: one wavefront per workgroup, so that a short list reaches more CUs (3,600 nodes 27 -> 12 us, 31,000
 // nodes 43 -> 33, 262,144 nodes 31 -> 33)
 constexpr int MASS_BLOCK = 64, MASS_GRID = FS_GRID * FS_BLOCK / MASS_BLOCK;
-// Passes between two orderings of the interface list (k_fs_build_list). us a cycle over 200 cycles, every pass / 8 / 32 /
-// never: 262,144 interface nodes of 512 x 512 x 256 1580 to 1593 / 1565 to 1583 / 1566 to 1591 / 1569 to 1656 and
-// rising, 31,000 of 384 x 128 x 192 336 / 319 / 316 / 316, 3,600 of 101 x 47 x 66 149 / 146 / 146 / 143.
+// Passes between two orderings of the interface list (k_fs_build_list). us a cycle after some 1,000 cycles, every pass / 8 /
+// 16 / 32 / never: 262,144 interface nodes of 512 x 512 x 256 1670 / 1664 / 1667 / 1675 / 1896, 31,000 of 384 x 128 x 192 445
+// / 426 / 428 / 430 / 443, 3,600 of 101 x 47 x 66 159 / 155 / 156 / 155 / 157. 8 and 16 are within the runs of one side.
 constexpr uint32_t SORT_STEPS = 16;
 enum : uint8_t { FS_STAY = 0, FS_FILLED = 1, FS_EMPTIED = 2 };
 

@@ -101,10 +101,11 @@ __device__ __forceinline__ bool lane_coord(const LBKParams& p, Coord& c) {
 }
 
 // Whether an inactive lane stores populations with the active ones of its wavefront: where the 128-byte line of its
-// node holds an active node, so that the line is written whole. Nothing reads an inactive node's populations. A line
-// written in part costs the memory a read as well: the ghost layers at both ends of a row alone made the FP32 step of
-// 256^3 nodes 562 us instead of 465, of 64 x 150 x 150 nodes 79 instead of 47. The stores of both kinds of lanes
-// are the same instructions (stores of their own for the inactive lanes made FP64 steps 13 to 40 % slower than none).
+// node holds an active node, so that the line is written whole. Nothing reads an inactive node's populations. Lines
+// written in part cost far more than their bytes: the ghost layers at both ends of a row alone made the FP32 step of
+// 256^3 nodes 562 us instead of 465, of 64 x 150 x 150 nodes 79 instead of 47, while the L2's counted traffic is about
+// the same (256^3: 1.53 GB read and 1.21 written with them, 1.47 and 1.31 without; what happens behind it isn't
+// counted). The stores of both kinds of lanes are the same instructions (stores of their own for the inactive lanes made FP64 steps 13 to 40 % slower than none).
 // All lanes of the wavefront that hold a node take part.
 template <typename T>
 __device__ __forceinline__ bool fills_line(bool act) {

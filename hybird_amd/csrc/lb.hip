@@ -1168,7 +1168,8 @@ __global__ void k_fill_u32(uint32_t* __restrict__ a, uint32_t v, size_t n) {
         return;                                                                                                    \
     }
 // Cylinders (p.curvw set, CUR = true): the curved-wall pull and the capture of
-// every active node's density and velocity for the next step's curved links.
+// every active node's density and velocity for the next step's curved links. They take the row map at every row length
+// (the other one wasn't measured with them).
 #define HYB_FUSED_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, false, false)
 #define HYB_MERGE_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, false, true)
 #define HYB_CURVED_CASE(PULL, VV, CO) HYB_FUSED_LAUNCH(PULL, VV, CO, true, false)
