@@ -28,6 +28,8 @@ enum ElemField : int {
     EF_COUNT = 159
 };
 
+constexpr int MAX_WALLS = 8;  // the six box planes and DRUM's two y walls
+
 struct DEMParams {
     int P;                 // standard particles: the spheres of all elements (elements with size > 1 hold several)
     int E;                 // elements
@@ -37,7 +39,7 @@ struct DEMParams {
     int npbc, nwalls;
     int nobj;              // objects (originals and periodic copies), DEMBuffers::objs
     PbcDev pbc[3];
-    WallDev walls[6];
+    WallDev walls[MAX_WALLS];
     double cellWidth[3];
     unsigned nCells[3];
     double nebrRange, trigger, deltat;

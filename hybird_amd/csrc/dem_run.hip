@@ -290,7 +290,7 @@ struct Cold {
     double I[LANES], dI[LANES];                    // I[c] and I[c+1] - I[c+2] (newtonAcc)
     uint2 nb[ENT_LANE][LANES];                     // partner and its ghost's period signs
     double c1[5], c2[5], co1[6], co2[6], demF[3];  // from DEMParams (as kernel arguments they are spilled)
-    double period[3], wall[8][6];                  // periods along the axes (0: none); normal and point of each wall
+    double period[3], wall[MAX_WALLS][6];          // periods along the axes (0: none); normal and point of each wall
 };
 
 template <int LANES>
@@ -903,7 +903,7 @@ __global__ void __launch_bounds__(ONE && !CL ? 512 : 256, ONE && CL ? 1 : 2) k_d
             if (g.pbc[k].v.y != 0.0) K.period[1] = g.pbc[k].v.y;
             if (g.pbc[k].v.z != 0.0) K.period[2] = g.pbc[k].v.z;
         }
-        for (int k = 0; k < p.nwalls && k < 8; ++k) {
+        for (int k = 0; k < p.nwalls; ++k) {
             const WallDev& w = g.walls[k];
             K.wall[k][0] = w.n.x; K.wall[k][1] = w.n.y; K.wall[k][2] = w.n.z;
             K.wall[k][3] = w.p.x; K.wall[k][4] = w.p.y; K.wall[k][5] = w.p.z;
